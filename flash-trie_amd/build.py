@@ -109,6 +109,7 @@ def build(verbose=False):
     bid = ["-DFT_BUILD_ID=\"" + source_id() + "\""]
     hip_objs = {
         "tbs_kernel.hip": os.path.join(OBJ, "tbs_kernel.o"),
+        "sort_rows.hip": os.path.join(OBJ, "sort_rows.o"),
         "ft_runtime.cpp": os.path.join(OBJ, "ft_runtime.o"),
     }
     host_objs = {

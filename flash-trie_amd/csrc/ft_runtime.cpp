@@ -1034,6 +1034,7 @@ struct PackState {
   double s_lo = 0.0, s_hi = 0.0;  // bounds of the parent scores at the next row
   uint32_t rk_planned = 0;        // where the row indices go when a row needs them
   bool rk_used = false;
+  bool raw = false;  // rows are left in the caller's order (sorted on the device)
 };
 
 static int pack_head(const ft_request& q, size_t r, DevReq& d, uint8_t* base, PackState& ps,
@@ -1049,7 +1050,7 @@ static int pack_head(const ft_request& q, size_t r, DevReq& d, uint8_t* base, Pa
              FT_E_INPUT;
   }
   std::memcpy(base + d.beams_off, q.beams, 4ull * T);
-  ps = PackState();
+  ps = PackState{0.0, 0.0, 0u, false, ps.raw};
   // d.rk_off holds the planned offset of the indices until a row needs them
   ps.rk_planned = d.rk_off;
   return FT_OK;
@@ -1083,7 +1084,9 @@ static int pack_rows(const ft_request& q, size_t r, const DevReq& d, uint8_t* ba
     uint16_t* ok = rk_s + (uint64_t)t * K;
     const RowScan sc = g_scan_row(rid, rlp, K, q.token_logp_threshold, oid, olp);
     if (sc.bad) return *err = who() + "topk_logp holds NaN or +inf", FT_E_INPUT;
-    if (sc.sorted) {
+    if (ps.raw) {
+      // (copied as they came, by the scan)
+    } else if (sc.sorted) {
       if (ps.rk_used)
         for (uint32_t k = 0; k < K; ++k) ok[k] = (uint16_t)k;
     } else {
@@ -1627,6 +1630,46 @@ void pack_stream(PackJob& j, std::pair<uint32_t, uint32_t>* tmp) {
 }
 }  // namespace
 
+namespace {
+// Whether a batch's rows are sorted on the device: some request's first row
+// is out of token order, and every row fits the sort.  The first rows alone
+// decide, at a few compares a request (rows that come by score are out of
+// order within the first few proposals); a batch whose disorder starts later
+// is sorted on the packing thread.  Against that sort (19 us a row of 777)
+// the device pays one launch, ~10 us, at any number of rows.
+bool sorts_on_device(const ft_request* reqs, size_t batch, const StagedReq* staged) {
+  bool raw = false;
+  for (size_t r = 0; r < batch; ++r) {
+    if (staged[r].skip) continue;
+    const uint32_t K = staged[r].K;
+    if (K > kMaxLdsTopk) return false;
+    const uint32_t* id = reqs[r].topk_id_rows ? reqs[r].topk_id_rows[0] : reqs[r].topk_id;
+    for (uint32_t k = 1; id && !raw && k < K; ++k) raw = id[k] <= id[k - 1];
+  }
+  return raw;
+}
+
+// Packs every request of `j` with its rows as they came, and writes its ready
+// word (final: the launch follows).
+void pack_raw(PackJob& j, std::pair<uint32_t, uint32_t>* tmp) {
+  for (size_t r = 0; r < j.batch; ++r) {
+    if (j.staged[r].skip) continue;
+    const DevReq& d = j.D[r];
+    PackState ps;
+    ps.raw = true;
+    uint8_t* base = j.H + d.in_off;
+    int rc = pack_head(j.reqs[r], r, j.D[r], base, ps, &j.msg[r]);
+    if (!rc) rc = pack_rows(j.reqs[r], r, d, base, 0, d.T, tmp, ps, &j.msg[r]);
+    j.rc[r] = rc;
+    __atomic_store_n(&j.ready[r],
+                     j.tag | (rc ? (unsigned long long)kReadyWithdrawn
+                                 : ((unsigned long long)d.T << kReadyRowsShift) | kReadyOk | kReadyRk),
+                     __ATOMIC_RELEASE);
+  }
+  _mm_sfence();
+}
+}  // namespace
+
 // A streamed search: the kernel is launched as soon as the batch's shapes
 // are checked and laid out, and the requests are packed into mapped host
 // memory while it runs.  A request's leader starts once the request's
@@ -1705,7 +1748,15 @@ int ft_search_each(ft_ctx* c, const ft_request* reqs, size_t batch, ft_result* r
   // the result headers start unpublished
   for (size_t r = 0; r < batch; ++r)
     __atomic_store_n(&((OutHeader*)(c->h_out + c->out_stride * r))->status, 0u, __ATOMIC_RELAXED);
-  if (int rc = launch_timed(c, a, false)) return drop(rc);
+  const bool raw = sorts_on_device(reqs, batch, c->staged.data());
+  if (raw) {
+    a.stage_src = nullptr;
+    a.sort_src = c->m_stage;
+    a.sort_topk = kmax;
+    for (size_t i = 0; i < batch; ++i) a.sort_steps = std::max(a.sort_steps, c->staged[i].T);
+  } else if (int rc = launch_timed(c, a, false)) {
+    return drop(rc);
+  }
   PackJob job;
   job.reqs = reqs;
   job.D = D;
@@ -1718,7 +1769,12 @@ int ft_search_each(ft_ctx* c, const ft_request* reqs, size_t batch, ft_result* r
   job.rc.assign(batch, FT_OK);
   job.msg.resize(batch);
   if (c->pack_delay_us) std::this_thread::sleep_for(std::chrono::microseconds(c->pack_delay_us));
-  pack_stream(job, c->sort_tmp.data());
+  if (raw) {
+    pack_raw(job, c->sort_tmp.data());
+    if (int rc = launch_timed(c, a, false)) return drop(rc);
+  } else {
+    pack_stream(job, c->sort_tmp.data());
+  }
   // Each request's results once its leader has published them (kStatusDone
   // in its header, written last with a system-scope release), in the order
   // the requests finish; the stream is looked at now and then, so that a
@@ -1741,6 +1797,13 @@ int ft_search_each(ft_ctx* c, const ft_request* reqs, size_t batch, ft_result* r
     --left;
     if (job.rc[r]) return;  // withdrawn: its packing error is reported
     const OutHeader* oh = (const OutHeader*)(c->h_out + c->out_stride * r);
+    if (raw && !c->staged[r].skip && (oh->status & kStatusWithdrawn)) {
+      // the sort met a token twice: the host's own packing says which (the
+      // search reads nothing of h_stage any more)
+      job.rc[r] = pack_request(reqs[r], r, D[r], c->h_stage + D[r].in_off, c->sort_tmp.data(),
+                               &job.msg[r]);
+      if (job.rc[r]) return;
+    }
     if (!c->staged[r].skip && (oh->status & kStatusNotReady)) {
       retry.push_back(r);
       return;

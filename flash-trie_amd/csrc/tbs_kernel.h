@@ -334,6 +334,13 @@ struct KArgs {
   const RootEnt* root_dir;
   uint32_t root_n;
   uint32_t root_force;
+  // streamed search of rows in no token order (null otherwise): the batch's
+  // blocks were packed as they came, at sort_src (mapped host memory), before
+  // the launch; launch_sort_rows puts them in order into `stage` first (rows
+  // of up to sort_topk proposals, requests of up to sort_steps of them), and
+  // the search copies nothing (stage_src is null)
+  const uint8_t* sort_src;
+  uint32_t sort_topk, sort_steps;
 };
 
 // LOUDS directory of the trie's shape: for every node v in breadth-first
@@ -355,6 +362,10 @@ constexpr uint32_t kLoudsBlockBits = 512;
 // stop times: events attached to its dispatch, not markers around it)
 hipError_t launch_tbs(const KArgs& args, hipStream_t stream, hipEvent_t start = nullptr,
                       hipEvent_t stop = nullptr);
+
+// Sorts the rows of a streamed batch from args.sort_src into args.stage (see
+// sort_rows.hip), on `stream`; launch_tbs does it in front of such a search.
+hipError_t launch_sort_rows(const KArgs& args, hipStream_t stream);
 
 // Fills the root directory `dir` (root_n entries, zeroed by the caller)
 // from the root's `deg` children starting at node c0, on `stream`.  `args`

@@ -1549,6 +1549,10 @@ __device__ __forceinline__ bool stage_in(const KArgs& a, uint32_t req, const Dev
     }
     return false;
   }
+  if (a.stage_src == nullptr) {  // the whole batch was sorted into the stage
+    ss = StageState{d.T, d.T, split, true, true, false};
+    return true;
+  }
   ss = StageState{0u, 0u, split, false, false, false};
   stage_rows<8>(a, d, true, 0u, final ? d.T : split, v, ss);
   return true;
@@ -1669,7 +1673,7 @@ __device__ __forceinline__ void helper_loop(const KArgs& a, const DevReq& d, uin
   const uint32_t* rid = (const uint32_t*)(in + d.rid_off);
   const float* rlp = (const float*)(in + d.rlp_off);
   if constexpr (kStreamed) {
-    if (g == 1) helper_copy(a, blockIdx.x % a.batch, d, ws, sm);
+    if (g == 1 && a.stage_src != nullptr) helper_copy(a, blockIdx.x % a.batch, d, ws, sm);
   }
   // The helpers that share the leader's XCD (blocks are dealt to the 8 XCDs
   // in turn: block req + g * batch sits with the leader's when g * batch is
@@ -1872,7 +1876,7 @@ __device__ __forceinline__ void helper_loop(const KArgs& a, const DevReq& d, uin
     if (g == pfg && t + 2u < d.T && !big) {
       bool ready = true;
       if constexpr (kStreamed) {
-        if (stream_split(a.head_rows, d.T, d.K) < d.T) {
+        if (a.stage_src != nullptr && stream_split(a.head_rows, d.T, d.K) < d.T) {
           const unsigned long long c = ld_relaxed(&ctl->copy);
           ready = (c >> 32) == a.epoch && ((uint32_t)c & kCopyDone);
         }
@@ -3224,6 +3228,10 @@ hipError_t clear_controls(uint8_t* ws, uint64_t stride, uint64_t ctl_off, uint64
 hipError_t launch_tbs(const KArgs& args, hipStream_t stream, hipEvent_t start,
                       hipEvent_t stop) {
   const dim3 grid(args.batch * args.wgs), block(kBlock);
+  if (args.sort_src) {
+    const hipError_t e = launch_sort_rows(args, stream);
+    if (e != hipSuccess) return e;
+  }
   if (args.louds_words) {
     if (args.ready) return hipErrorInvalidValue;  // (no streamed LOUDS search)
     hipExtLaunchKernelGGL((tbs_kernel<true, false>), grid, block, 0, stream, start, stop, 0,
