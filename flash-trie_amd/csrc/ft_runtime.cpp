@@ -128,6 +128,7 @@ struct ft_ctx {
   uint32_t wgs_req = 4096;    // workgroups per request (clamped to residency:
                               // a lone request gets every CU)
   uint32_t share_min = 4096;  // work items from which a step is shared
+  uint64_t sort_min = 2048;   // proposals from which a batch is sorted on the device
   // a streamed search publishes each request's first head_rows rows before
   // it packs the rest of any (0: whole requests); helper 1 of the request
   // copies the rest to the device while the leader searches
@@ -767,6 +768,10 @@ int ft_create(const void* image, size_t image_bytes, int device,
   if (const char* s = std::getenv("FT_SHARE_MIN")) {
     const long v = std::strtol(s, nullptr, 10);
     if (v >= 0) c->share_min = (uint32_t)v;
+  }
+  if (const char* s = std::getenv("FT_SORT_MIN")) {
+    const long v = std::strtol(s, nullptr, 10);
+    if (v >= 0) c->sort_min = (uint64_t)v;
   }
   if (const char* s = std::getenv("FT_TEST_NO_CLAIMS")) c->no_claims = std::atoi(s) ? 1u : 0u;
   if (const char* s = std::getenv("FT_SCAN_MULT")) {
@@ -1632,21 +1637,29 @@ void pack_stream(PackJob& j, std::pair<uint32_t, uint32_t>* tmp) {
 
 namespace {
 // Whether a batch's rows are sorted on the device: some request's first row
-// is out of token order, and every row fits the sort.  The first rows alone
-// decide, at a few compares a request (rows that come by score are out of
-// order within the first few proposals); a batch whose disorder starts later
-// is sorted on the packing thread.  Against that sort (19 us a row of 777)
-// the device pays one launch, ~10 us, at any number of rows.
-bool sorts_on_device(const ft_request* reqs, size_t batch, const StagedReq* staged) {
+// is out of token order within its first kSortLook proposals, and every row
+// fits the sort.  A few compares a request decide, because the launch of a
+// batch in order waits for them (all of the first rows took 33 us of a batch
+// of 64): rows that come by score are out of order within the first few
+// proposals.  A batch whose disorder starts later is sorted on the packing
+// thread.  Against that sort (19 us a row of 777) the device pays one launch,
+// ~10 us, at any number of rows: calls with 2048 proposals in all take 107 us
+// with the thread's sort and 101 with the device's (rows of 256), with 1536
+// 104 and 110 (rows of 128); sort_min is the least that the device takes.
+constexpr uint32_t kSortLook = 32;
+bool sorts_on_device(const ft_request* reqs, size_t batch, const StagedReq* staged,
+                     uint64_t sort_min) {
   bool raw = false;
+  uint64_t proposals = 0;
   for (size_t r = 0; r < batch; ++r) {
     if (staged[r].skip) continue;
     const uint32_t K = staged[r].K;
     if (K > kMaxLdsTopk) return false;
+    proposals += (uint64_t)staged[r].T * K;
     const uint32_t* id = reqs[r].topk_id_rows ? reqs[r].topk_id_rows[0] : reqs[r].topk_id;
-    for (uint32_t k = 1; id && !raw && k < K; ++k) raw = id[k] <= id[k - 1];
+    for (uint32_t k = 1; id && !raw && k < std::min(K, kSortLook); ++k) raw = id[k] <= id[k - 1];
   }
-  return raw;
+  return raw && proposals >= sort_min;
 }
 
 // Packs every request of `j` with its rows as they came, and writes its ready
@@ -1748,7 +1761,7 @@ int ft_search_each(ft_ctx* c, const ft_request* reqs, size_t batch, ft_result* r
   // the result headers start unpublished
   for (size_t r = 0; r < batch; ++r)
     __atomic_store_n(&((OutHeader*)(c->h_out + c->out_stride * r))->status, 0u, __ATOMIC_RELAXED);
-  const bool raw = sorts_on_device(reqs, batch, c->staged.data());
+  const bool raw = sorts_on_device(reqs, batch, c->staged.data(), c->sort_min);
   if (raw) {
     a.stage_src = nullptr;
     a.sort_src = c->m_stage;

@@ -17,8 +17,10 @@ def trie(ft, po):
     toks, offs = ft.synth_keys(30000, VOCAB, 2, 5, 0.6, 3)
     t = ft.Trie()
     t.build_arrays(toks, offs)
-    t.init_tbs_gpu(4, max_num_topk=4097, max_num_outpos=4, max_num_out_beams=48,
-                   max_num_out_tokens=48 * 4, max_num_inter_beams=4096)
+    with pytest.MonkeyPatch.context() as m:  # the small rows on the device too
+        m.setenv("FT_SORT_MIN", "0")
+        t.init_tbs_gpu(4, max_num_topk=4097, max_num_outpos=4, max_num_out_beams=48,
+                       max_num_out_tokens=48 * 4, max_num_inter_beams=4096)
     return t, po.OracleTrie.from_keys(toks=toks, offs=offs)
 
 
