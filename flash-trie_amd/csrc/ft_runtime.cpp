@@ -129,6 +129,8 @@ struct ft_ctx {
                               // a lone request gets every CU)
   uint32_t share_min = 4096;  // work items from which a step is shared
   uint64_t sort_min = 2048;   // proposals from which a batch is sorted on the device
+  uint32_t cut_pairs = 160;   // see KArgs::cut_pairs
+  bool lean = true;           // false: the general instantiation at any size
   // a streamed search publishes each request's first head_rows rows before
   // it packs the rest of any (0: whole requests); helper 1 of the request
   // copies the rest to the device while the leader searches
@@ -373,7 +375,8 @@ static int build_labels(ft_ctx* c, const uint8_t* image) {
   }
   if (bad) return fail(FT_E_IMAGE, "ft_create: token ids must be below 2^31 - 1");
   hipError_t e;
-  if ((e = hipMalloc(&c->d_labels, N * sizeof(uint32_t))) != hipSuccess)
+  // (one word past the last label: the kernel reads labels in aligned pairs)
+  if ((e = hipMalloc(&c->d_labels, (N + 1) * sizeof(uint32_t))) != hipSuccess)
     return hip_fail(e, "hipMalloc(labels)");
   if ((e = hipMemcpy(c->d_labels, lab.get(), N * sizeof(uint32_t),
                      hipMemcpyHostToDevice)) != hipSuccess)
@@ -490,7 +493,7 @@ static int build_wide_index(ft_ctx* c, const uint8_t* image) {
   // uninitialised: every table is cleared by the thread that fills it
   std::unique_ptr<WideBucket[]> tab(new (std::nothrow) WideBucket[buckets]);
   if (!tab) return fail(FT_E_NOMEM, "wide-node index: host memory");
-  std::vector<uint8_t> failed(ent.size(), 0);
+  std::vector<uint8_t> failed(ent.size(), 0), closes(ent.size(), 0);
   {
     std::atomic<size_t> next{0};
     std::vector<std::thread> th;
@@ -512,6 +515,7 @@ static int build_wide_index(ft_ctx* c, const uint8_t* image) {
             const uint32_t elen = (meta >> FT_META_ELEN_SHIFT) & FT_META_ELEN_MASK;
             const bool sel = (meta & FT_META_TERMINAL) && elen == 1;
             const uint32_t tokw = (R[ch].first_tok & kTokMask) | (sel ? kSlotSel : 0u);
+            if (sel) closes[i] = 1;
             // tokens that do not fit the slot word: no table for this node
             if (R[ch].first_tok >= kSlotEmptyTok ||
                 !cuckoo_insert(tb, e.log2nb, tokw, ch, &rng)) {
@@ -549,7 +553,8 @@ static int build_wide_index(ft_ctx* c, const uint8_t* image) {
     const long v = std::strtol(fe, nullptr, 10);
     if (v >= 0 && v <= 32) fp_max = (uint32_t)v;
   }
-  for (auto& e : ent) e.flags = e.log2nb <= fp_max ? kWideFiltered : 0u;
+  for (size_t i = 0; i < ent.size(); ++i)
+    ent[i].flags = (ent[i].log2nb <= fp_max ? kWideFiltered : 0u) | (closes[i] ? 0u : kWideOpen);
   uint64_t n_ok = 0;
   for (size_t i = 0; i < ent.size(); ++i) n_ok += failed[i] ? 0 : 1;
   // directory groups, load <= 1/2
@@ -768,6 +773,11 @@ int ft_create(const void* image, size_t image_bytes, int device,
   if (const char* s = std::getenv("FT_SHARE_MIN")) {
     const long v = std::strtol(s, nullptr, 10);
     if (v >= 0) c->share_min = (uint32_t)v;
+  }
+  if (const char* s = std::getenv("FT_LEAN")) c->lean = std::atoi(s) != 0;
+  if (const char* s = std::getenv("FT_CUT_PAIRS")) {
+    const long v = std::strtol(s, nullptr, 10);
+    if (v >= 0 && v < 1000000) c->cut_pairs = (uint32_t)v;
   }
   if (const char* s = std::getenv("FT_SORT_MIN")) {
     const long v = std::strtol(s, nullptr, 10);
@@ -1327,7 +1337,8 @@ int ft_stage(ft_ctx* c, const ft_request* reqs, size_t batch) {
 // at `stage` (DevReq array first), with workspace slots of `ws_stride`
 // bytes from `ws` and output blocks of `out_stride` bytes from `out`.
 static KArgs kernel_args(const ft_ctx* c, const uint8_t* stage, size_t first, size_t count,
-                         uint32_t kmax, uint8_t* ws, uint64_t ws_stride, const WsLayout& lay,
+                         uint32_t kmax, uint64_t bmax, uint8_t* ws, uint64_t ws_stride,
+                         const WsLayout& lay,
                          uint8_t* out, uint64_t out_stride) {
   KArgs a{};
   a.recs = (const ft_node_rec*)(c->d_image + c->hdr.recs_offset);
@@ -1347,6 +1358,14 @@ static KArgs kernel_args(const ft_ctx* c, const uint8_t* stage, size_t first, si
   const uint32_t fit = (uint32_t)std::max<int>(1, c->max_resident / (int)count);
   a.wgs = std::max(1u, std::min(std::min(c->wgs_req, fit), lay.claim_slots));
   a.share_min = c->share_min;
+  a.cut_pairs = c->cut_pairs;
+  // the lean instantiation, where beams and rows fit it and the pairs of a step
+  // may be enough for its queue (at beam = K = 1000 from batch 2 on; on
+  // smaller batches and beams it gains nothing, and measured 0-2% slower)
+  a.lean = c->lean && kmax <= kBlockThreads && bmax <= kBlockThreads &&
+                   bmax * kmax > (uint64_t)kQueueMinChunks * kBlockThreads * a.wgs
+               ? 1u
+               : 0u;
   uint32_t ep = ++g_launch_epoch;
   if (ep == 0) ep = ++g_launch_epoch;
   a.epoch = ep;
@@ -1409,8 +1428,12 @@ int ft_launch_range(ft_ctx* c, size_t first, size_t count) {
                                 std::to_string(count) + ") exceeds the staged requests or max_batch_size " +
                                 std::to_string(c->max_batch));
   uint32_t kmax = 1;
-  for (size_t i = first; i < first + count; ++i) kmax = std::max(kmax, c->staged[i].K);
-  const KArgs a = kernel_args(c, c->d_stage, first, count, kmax, c->d_ws, c->ws_stride,
+  uint64_t bmax = 1;
+  for (size_t i = first; i < first + count; ++i) {
+    kmax = std::max(kmax, c->staged[i].K);
+    bmax = std::max(bmax, c->staged[i].bmax);
+  }
+  const KArgs a = kernel_args(c, c->d_stage, first, count, kmax, bmax, c->d_ws, c->ws_stride,
                               c->lay, c->d_out, c->out_stride);
   if (int rc = launch_timed(c, a, true)) return rc;
   c->launched = true;
@@ -1749,8 +1772,12 @@ int ft_search_each(ft_ctx* c, const ft_request* reqs, size_t batch, ft_result* r
     return drop(fail(rc, msg));
   }
   uint32_t kmax = 1;
-  for (size_t i = 0; i < batch; ++i) kmax = std::max(kmax, c->staged[i].K);
-  KArgs a = kernel_args(c, c->d_stage, 0, batch, kmax, c->d_ws, c->ws_stride, c->lay, c->d_out,
+  uint64_t bmax = 1;
+  for (size_t i = 0; i < batch; ++i) {
+    kmax = std::max(kmax, c->staged[i].K);
+    bmax = std::max(bmax, c->staged[i].bmax);
+  }
+  KArgs a = kernel_args(c, c->d_stage, 0, batch, kmax, bmax, c->d_ws, c->ws_stride, c->lay, c->d_out,
                         c->out_stride);
   a.reqs = (const DevReq*)c->m_stage;
   a.stage_src = c->m_stage;
@@ -1973,7 +2000,7 @@ int ft_search_noalloc(ft_ctx* c, const ft_request* reqs, size_t batch,
   if ((e = clear_controls(base + ws_off, ws_stride, L.ctl, L.claims, L.dones, L.claim_slots,
                           (uint32_t)batch, c->stream)) != hipSuccess)
     return hip_fail(e, "clear_controls");
-  const KArgs a = kernel_args(c, base, 0, batch, (uint32_t)K, base + ws_off, ws_stride, L,
+  const KArgs a = kernel_args(c, base, 0, batch, (uint32_t)K, B, base + ws_off, ws_stride, L,
                               base + out_off, out_stride);
   if (int rc = launch_timed(c, a, false)) return rc;
   if ((e = hipMemcpyAsync(g_na_out, base + out_off, out_stride * batch, hipMemcpyDeviceToHost,

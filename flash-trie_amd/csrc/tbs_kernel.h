@@ -16,6 +16,12 @@ constexpr uint32_t kMaxTopk = 65535;
 // Parent index and proposal index are packed into 16 bits each.
 constexpr uint32_t kMaxBeams = 65535;
 constexpr uint32_t kNoHist = 0xFFFFFFFFu;
+// Threads of the search kernel's workgroups: the longest beam and row of its
+// lean instantiation.
+constexpr uint32_t kBlockThreads = 1024;
+// A step is queued (queues_items) when its 64-item chunks are more than this
+// many for each wave of its workgroups.
+constexpr uint32_t kQueueMinChunks = 4;
 
 enum : uint32_t { kReqEarlyExit = 1u, kReqSkip = 2u };
 
@@ -174,7 +180,7 @@ struct WideDir {        // one node's table (host side)
   uint32_t node;
   uint32_t log2nb;      // log2 of the bucket count (>= 1)
   uint32_t bucket_off;  // first bucket of the node's table
-  uint32_t flags;       // kWideFiltered
+  uint32_t flags;       // kWideFiltered, kWideOpen
 };
 constexpr uint32_t kDirSlots = 4;
 struct WideDirGroup {   // kDirSlots directory entries (device side)
@@ -185,6 +191,8 @@ struct WideDirGroup {   // kDirSlots directory entries (device side)
 };
 static_assert(sizeof(WideDirGroup) == 64, "WideDirGroup layout");
 constexpr uint32_t kWideFiltered = 1u;
+// no child of the node closes a key one token below it (no slot has kSlotSel)
+constexpr uint32_t kWideOpen = 2u;
 constexpr uint32_t kFpMaxLog2 = 16;
 
 // Root directory: the root's children indexed by their first token, one
@@ -211,6 +219,7 @@ constexpr uint32_t kRdLink = 2u;      // a link parent at step 1
 constexpr uint32_t kRdTable = 4u;     // has a hash table
 constexpr uint32_t kRdFiltered = 8u;  // ... with fingerprint filtering
 constexpr uint32_t kRdErr = 16u;      // its entry could not be built
+constexpr uint32_t kRdOpen = 32u;     // ... with kWideOpen
 // Largest directory built (entries); a root with larger child tokens keeps
 // its hash table or binary search.
 constexpr uint32_t kRootDirMax = 1u << 25;
@@ -260,11 +269,14 @@ struct Ctl {
   // streamed search: (launch epoch << 32) | 1 once the leader has copied
   // the request's first rows to the device stage
   unsigned long long head;
-  unsigned long long pad4;
+  // the shared step's cut of its `next` pushes (see cut_of_step): the norm's
+  // order-preserving key, and which pushes the round takes (kCut*)
+  unsigned long long cut;
   // streamed search: the copy of the rows after the first ready word's
   // (launch epoch << 32) | kCopy* state, claimed by helper 1 or the leader
   unsigned long long copy;
-  uint32_t pad3[16];
+  uint32_t cut_mode;
+  uint32_t pad3[15];
 };
 static_assert(sizeof(Ctl) == 384, "Ctl layout");
 
@@ -304,6 +316,12 @@ struct KArgs {
   uint32_t wgs;        // workgroups per request (1 leader + wgs-1 helpers)
   uint32_t share_min;  // work items from which a step is shared
   uint32_t epoch;      // launch counter (tags the control words)
+  // (parent, proposal) pairs a kept hypothesis that a shared step's cut lets
+  // through (cut_of_step); 0: no cuts
+  uint32_t cut_pairs;
+  // every beam width and K of the launch is at most the kernel's block and a
+  // step may have enough items for its queue: the lean instantiation runs
+  uint32_t lean;
   // helpers never claim their slices (a test of the leader's take-over of
   // unclaimed slices; never set otherwise)
   uint32_t no_claims;

@@ -47,7 +47,7 @@
 
 namespace ftk {
 
-constexpr int kBlock = 1024;
+constexpr int kBlock = (int)kBlockThreads;
 constexpr int kWaves = kBlock / 64;
 // selection: bins of the first histogram and the keys one bin may hold in LDS
 constexpr int kWideBits = 11;
@@ -63,6 +63,15 @@ constexpr int kRowHashLog2 = 12;
 constexpr int kRowHash = 1 << kRowHashLog2;
 constexpr uint32_t kRowHashMaxK = kRowHash / 2;
 constexpr uint32_t kRowHashEmpty = 0xFFFFFFFFu;
+// beside it one bit per token of the row, in kRowBits bits by the same hash:
+// a label whose bit is clear is not in the row
+constexpr int kRowBitsLog2 = 15;
+constexpr uint32_t kRowBits = 1u << kRowBitsLog2;
+// expansion: chunks of work items whose filter words a wave reads at once,
+// and the items it holds that passed the filters (at most 63 left over and
+// those of these chunks)
+constexpr uint32_t kQueueChunks = 1;
+constexpr uint32_t kQueueCap = 64u * (kQueueChunks + 1u);
 // the leader hashes the row for steps of at least this many work items (a
 // smaller step does too few lookups to repay the build)
 constexpr uint32_t kRowHashMinWork = 2048;
@@ -86,9 +95,14 @@ struct alignas(16) Smem {
   uint32_t n_next, n_sel, n_out, overflow;
   uint32_t status;
   unsigned long long cnt_parents, cnt_children, cnt_probes;
+  // thread 0's of the leader: its clocks and the candidates so far (here
+  // rather than in registers through the steps)
+  unsigned long long t_exp, t_sel, t_all0, t_post, t_wait, n_cands;
   unsigned long long bcast;
   uint32_t hstep[7];  // a helper's view of the posted step (+ whether it
                       // took its slice)
+  unsigned long long hcut;  // ... and its cut
+  uint32_t hcut_mode;
   uint32_t lead_flag;   // the leader's broadcast of a decision of thread 0
   uint32_t n_stolen;    // helper slices the leader took over this step
   uint16_t stolen[256];
@@ -122,6 +136,8 @@ struct alignas(16) Smem {
   uint8_t p_mode[kBlock];
   // link parents (kNoCursor otherwise): index in tail[] of the pending token
   uint32_t p_lp[kBlock];
+  // expansion: the row's token bits (see kRowBits)
+  uint32_t rh_bits[kRowBits / 32];
   // the leader's own per-parent data for its emit, which overwrites the
   // table above with the next step's, copied by the parent phase: score,
   // history record and, for a link parent that stays one on its own edge,
@@ -137,6 +153,9 @@ struct alignas(16) Smem {
     struct {
       uint32_t rh_tok[kRowHash];
       uint16_t rh_pos[kRowHash];
+      // the items that passed the filters, per wave: kPk* | parent << 16 |
+      // item of the parent
+      uint32_t ex_queue[kWaves][kQueueCap];
     };
     // selection: positions of the kept candidates, and the keys and
     // positions of one histogram bin
@@ -214,6 +233,8 @@ constexpr uint32_t kModeMask = 0x0Fu;
 constexpr uint32_t kModeDepthOk = 0x80u;
 // a hashed parent whose table has fingerprint filtering (kWideFiltered)
 constexpr uint32_t kModeFiltered = 0x40u;
+// a hashed parent none of whose children closes a key (kWideOpen)
+constexpr uint32_t kModeOpen = 0x20u;
 
 enum : uint8_t {
   M_NONE = 0,
@@ -235,6 +256,9 @@ __device__ __forceinline__ uint64_t norm_key(double v) {
 __device__ __forceinline__ uint32_t lane_id() { return threadIdx.x & 63; }
 
 // whether some byte of v is zero
+__device__ __forceinline__ bool has_zero_byte(uint32_t v) {
+  return ((v - 0x01010101u) & ~v & 0x80808080u) != 0;
+}
 __device__ __forceinline__ bool has_zero_byte(uint64_t v) {
   return ((v - 0x0101010101010101ull) & ~v & 0x8080808080808080ull) != 0;
 }
@@ -348,6 +372,12 @@ __device__ __forceinline__ uint32_t block_excl_scan(uint32_t v, uint32_t* total,
   *total = sm.sel_cum;
   __syncthreads();
   return r;
+}
+
+// Adds to a counter in LDS without waiting for its value (the add returns
+// nothing), unlike += on it.
+__device__ __forceinline__ void lds_add(unsigned long long* p, unsigned long long x) {
+  (void)__hip_atomic_fetch_add(p, x, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
 }
 
 // Adds 1 to hist[digit] for every active lane; lanes of a wave that agree on
@@ -882,7 +912,8 @@ __device__ __forceinline__ ParEntry parent_entry(const KArgs& a, uint32_t node, 
         for (int k = 0; k < (int)kDirSlots; ++k) {
           if (nds[k] == node) {
             found = true;
-            e.mode = M_HASH | (((lgfs[k] >> 8) & kWideFiltered) ? kModeFiltered : 0u);
+            e.mode = M_HASH | (((lgfs[k] >> 8) & kWideFiltered) ? kModeFiltered : 0u) |
+                     (((lgfs[k] >> 8) & kWideOpen) ? kModeOpen : 0u);
             e.aux = lgfs[k] & 0xFFu;
             e.c0 = offs[k];
           }
@@ -921,7 +952,8 @@ __device__ __forceinline__ ParEntry root_child_entry(const KArgs& a, const uint4
     e.mode = M_SEARCH;
     e.work = K;
     if (f & kRdTable) {
-      e.mode = M_HASH | ((f & kRdFiltered) ? kModeFiltered : 0u);
+      e.mode = M_HASH | ((f & kRdFiltered) ? kModeFiltered : 0u) |
+               ((f & kRdOpen) ? kModeOpen : 0u);
       e.aux = (f >> 8) & 0xFFu;
       e.c0 = y.x;
     }
@@ -947,6 +979,9 @@ __device__ __forceinline__ uint32_t entry_work(uint32_t mode, uint32_t aux, uint
 
 __device__ __forceinline__ uint32_t row_hash(uint32_t tok) {
   return (tok * 0x9E3779B1u) >> (32 - kRowHashLog2);
+}
+__device__ __forceinline__ uint32_t row_bit(uint32_t tok) {
+  return (tok * 0x9E3779B1u) >> (32 - kRowBitsLog2);
 }
 
 // position of tok in the sorted LDS row, or -1: a probe or two when the row
@@ -1047,7 +1082,15 @@ struct StepView {
   uint32_t keep_lds_max;
   // every parent has exactly one work item (item w belongs to parent w)
   bool one_each;
+  // (queued) the round's cut of the `next` pushes
+  double cut;
+  uint32_t cut_mode;
 };
+
+// The cut of a shared step (cut_of_step).  kCutNone: every push.  kCutAbove:
+// the pushes into `next` whose norm is at least `cut`, and every one into
+// `selected`.  kCutBelow: the other pushes into `next`, none into `selected`.
+enum : uint32_t { kCutNone = 0u, kCutAbove = 1u, kCutBelow = 2u };
 
 // Position of tok in a sorted row held in the device stage (a row longer
 // than the LDS row arrays), or -1.  Device-coherent loads: a streamed
@@ -1059,6 +1102,96 @@ __device__ __forceinline__ int grow_find(const uint32_t* rid, uint32_t K, uint32
     if (ld_relaxed(rid + mid) < tok) lo = mid + 1; else hi = mid;
   }
   return (lo < K && ld_relaxed(rid + lo) == tok) ? (int)lo : -1;
+}
+
+// An item of the queued expansion: what it is -- a scanned child, a proposal
+// into a filtered table, an item with no filter, none -- then its parent
+// (kBlock of them at most) and its place among the parent's items.  kPkBit:
+// of a scanned child, its label is the upper one of its aligned pair; of a
+// queued proposal, its first fingerprint word matched.
+constexpr uint32_t kPkScan = 0u, kPkHash = 1u << 30, kPkAll = 2u << 30, kPkNone = 3u << 30;
+constexpr uint32_t kPkBit = 1u << 29, kPkItem = (1u << 26) - 1u;
+static_assert(kBlock <= 1024, "a parent index of the LDS table has 10 bits");
+
+// Queued expansion.  Few items survive the first look at them -- the row's
+// token bit of a scanned label, the fingerprint word of a hashed proposal
+// (one in seven over beam = K = 1000) -- while the work after it (the bucket,
+// the row position, scores, the append) is most of the instructions, and a
+// wave issues them all when a single lane of its chunk survives.  So each wave
+// runs the filters alone over its chunks, one 8-byte read an item, and queues
+// the survivors in LDS; the rest runs on 64 of them at a time.  Bound by the
+// device's rate of random lines from there: two or three chunks' reads in
+// flight a wave gained nothing.  Taken when a wave has more than four chunks
+// (beam = K = 1000, step 1 of 512K items over the 800M-key trie, without a cut:
+// 16 chunks a wave at batch 8, 54.5 -> 46.9 us; 126 at batch 64, 573 -> 510
+// us); with fewer there is nothing to gather, and the queue's own latency
+// shows (batch 1, two chunks: 19.0 -> 20.0 us).
+__device__ __forceinline__ bool queues_items(const KArgs& a, const StepView& v, uint32_t W,
+                                             uint32_t nwaves, bool hashed) {
+  return hashed && ((W + 63u) >> 6) > kQueueMinChunks * nwaves && a.scan_limit <= 65536u;
+}
+
+// Chooses the cut of a shared step whose items are queued.  Of the pushes into
+// `next` (19.7K of a step 1 at beam = K = 1000) only the M with the largest
+// norms survive, and most of the step's time goes into reads for the others:
+// the lookups of 372K hashed proposals, at the rate at which the device serves
+// random lines.  When at least M pushes have a norm >= cut, every push below it
+// loses (the M-th largest norm is >= cut, and neither the heap's content nor a
+// tie at its boundary depends on smaller norms), so the step first takes the
+// pushes from the cut up, without looking up the proposals that fall below it
+// (of parents whose children close no key: the others feed `selected` too),
+// and the leader checks their number; should fewer than M come, a second round
+// takes the rest.  The cut is the quantile of the scores of 64 x 64 sampled
+// (parent, proposal) pairs that lets cut_pairs * M pairs through: with 160, a
+// hit rate of 1 / 160 fills the beam in the first round, and the steps measured
+// have 1 / 110 to 1 / 30 (at beam = K = 1000, 5.1K pushes come).  Taken when
+// that is at most half of the pairs, and when the proposals that it can skip
+// are as many as those it lets through.  Step 1 at beam = K = 1000 over the
+// 800M-key trie: expansion 46.9 -> 41.5 and selection 25.1 -> 17.4 us at batch
+// 8, 510 -> 380 and 27.6 -> 18.1 us at batch 64.
+__device__ __forceinline__ void cut_of_step(const KArgs& a, StepView& v, uint32_t M,
+                                            const uint64_t* kbound, Smem& sm) {
+  const uint32_t tid = threadIdx.x;
+  const uint64_t pairs = (uint64_t)v.n_par * v.K, want = (uint64_t)a.cut_pairs * M;
+  const uint64_t klo = kbound[0], khi = kbound[1];
+  if (want == 0 || 2 * want > pairs || klo >= khi) return;
+  const uint32_t md = tid < v.n_par ? (uint32_t)sm.p_mode[tid] : 0u;
+  const bool skips =
+      (md & kModeMask) == M_HASH && ((md & kModeOpen) || !(md & kModeDepthOk));
+  if (tid < 16u) sm.hist[tid] = 0;
+  const uint32_t n_skips = (uint32_t)__syncthreads_count(skips);
+  if ((uint64_t)n_skips * v.K < want) return;
+  constexpr uint32_t kSide = 64, kPer = kSide * kSide / kBlock;
+  const double ps = sm.p_s[((tid & 63u) * v.n_par) / kSide];
+  double norm[kPer];
+#pragma unroll
+  for (uint32_t u = 0; u < kPer; ++u) {
+    const double x = (double)sm.row_lp[((tid >> 6) * kPer + u) * v.K / kSide];
+    const bool low = x <= (double)v.tok_thr || ps + x <= v.sent_thr;
+    norm[u] = low ? -__builtin_inf() : (ps + x) * v.lnf_next;
+  }
+  const uint32_t goal = max(1u, (uint32_t)(want * (kSide * kSide) / pairs));
+  auto value = [](uint64_t k) {  // the norm of a key
+    return __longlong_as_double((long long)((k >> 63) ? k & 0x7FFFFFFFFFFFFFFFull : ~k));
+  };
+  // the staged bounds hold every norm; 12 halvings of their range
+  double lo = value(klo), hi = value(khi);
+  bool found = false;
+#pragma unroll 1
+  for (uint32_t it = 0; it < 12u; ++it) {
+    const double mid = lo + 0.5 * (hi - lo);
+    uint32_t n = 0;
+#pragma unroll
+    for (uint32_t u = 0; u < kPer; ++u) n += (uint32_t)__popcll(__ballot(norm[u] >= mid));
+    if ((tid & 63u) == 0u) atomicAdd(&sm.hist[it], n);
+    __syncthreads();
+    const bool enough = sm.hist[it] >= goal;
+    found = found || enough;
+    if (enough) lo = mid; else hi = mid;
+  }
+  if (!found) return;
+  v.cut = lo;
+  v.cut_mode = kCutAbove;
 }
 
 // Expands the step's work items: each is (parent, child) for a scanned
@@ -1081,60 +1214,177 @@ __device__ __forceinline__ int grow_find(const uint32_t* rid, uint32_t K, uint32
 // step alone: its LDS counters are the list lengths and the control block is
 // not used (the counts stay in sm.lq_next, sm.lq_sel, sm.w_children and
 // sm.w_probes).
+// kLean (see tbs_kernel): the parent table and the row are in LDS, and a step
+// of many chunks is queued (queues_items).
+template <bool kLean>
 __device__ __forceinline__ void expand_range(const KArgs& a, const StepView& v, uint32_t W,
                              uint32_t gwave0, uint32_t nwaves, bool leader, bool solo,
                              bool hashed, Smem& sm) {
   const uint32_t tid = threadIdx.x, lane = tid & 63u;
-  const bool lds_par = v.n_par <= (uint32_t)kBlock;
+  const bool lds_par = kLean || v.n_par <= (uint32_t)kBlock;
+  const bool queued = kLean && queues_items(a, v, W, nwaves, hashed);
   uint32_t my_children = 0, my_probes = 0;
   const uint32_t K = v.K, t = v.t;
   const uint32_t nchunks = (W + 63u) >> 6;
   const uint32_t nwg = nwaves / (uint32_t)kWaves, slice = gwave0 / (uint32_t)kWaves;
-  for (uint32_t c = slice + nwg * (tid >> 6); c < nchunks; c += nwaves) {
-    const uint32_t w = (c << 6) + lane;
+  // The parents of chunk cc, when the table is in LDS: those of its first and
+  // last items (pa, pb - 1) by a 64-ary search of the prefix, two rounds of
+  // one LDS read a lane and a ballot (the prefix is non-decreasing, woff[0]
+  // is 0 and woff[n_par] is W, so each ballot is a run of low lanes); each
+  // lane then searches [pa, pb) alone -- nothing when one parent holds the
+  // whole chunk, as a hashed parent's K items mostly do.
+  auto chunk_parents = [&](uint32_t cc, uint32_t& pa, uint32_t& pb) {
+    const uint32_t w0 = cc << 6, wl = min(w0 + 63u, W - 1u);
+    const uint32_t st = (v.n_par + 64u) >> 6;  // 64 st > n_par
+    const uint32_t o1 = sm.woff[min(lane * st, v.n_par)];
+    const uint64_t m0 = __ballot(o1 <= w0), m1 = __ballot(o1 <= wl);
+    const uint32_t b0 = (63u - (uint32_t)__clzll((long long)m0)) * st;
+    const uint32_t b1 = (63u - (uint32_t)__clzll((long long)m1)) * st;
+    const uint32_t o2 = sm.woff[min(b0 + lane, v.n_par)];
+    const uint32_t o3 = sm.woff[min(b1 + lane, v.n_par)];
+    const uint64_t n0 = __ballot(lane < st && o2 <= w0);
+    const uint64_t n1 = __ballot(lane < st && o3 <= wl);
+    pa = b0 + (63u - (uint32_t)__clzll((long long)n0));
+    pb = b1 + (63u - (uint32_t)__clzll((long long)n1)) + 1u;
+  };
+  // (one value per wave: the loop's control stays in scalar registers)
+  uint32_t c = (uint32_t)__builtin_amdgcn_readfirstlane((int)(slice + nwg * (tid >> 6)));
+  uint32_t n_q = 0;
+  uint32_t* qd = sm.ex_queue[tid >> 6];
+  uint32_t p_at = 0;  // (queued) the first parent of the last chunk looked at
+  // (queued) the arrays the filters read, held: the kernel's arguments are
+  // otherwise loaded again, and waited for, in every round
+  const uint32_t* labels = a.labels;
+  const uint64_t* wfp = a.wfp;
+  if constexpr (kLean) asm volatile("" : "+s"(labels), "+s"(wfp));
+  for (;;) {
     bool do_next = false, do_sel = false;
     uint32_t cnode = 0, pj = 0, k = 0, tok = 0;
     double s2 = 0.0;
-    // The chunk's parents, when the table is in LDS: those of its first and
-    // last items (pa, pb) by a 64-ary search of the prefix, two rounds of one
-    // LDS read a lane and a ballot (the prefix is non-decreasing, woff[0] is
-    // 0 and woff[n_par] is W, so each ballot is a run of low lanes); each
-    // lane then searches [pa, pb] alone -- nothing when one parent holds the
-    // whole chunk, as a hashed parent's K items mostly do.
-    uint32_t pa = 0, pb = v.n_par;
-    if (lds_par && !v.one_each) {
-      const uint32_t w0 = c << 6, wl = min(w0 + 63u, W - 1u);
-      const uint32_t st = (v.n_par + 64u) >> 6;  // 64 st > n_par
-      const uint32_t o1 = sm.woff[min(lane * st, v.n_par)];
-      const uint64_t m0 = __ballot(o1 <= w0), m1 = __ballot(o1 <= wl);
-      const uint32_t b0 = (63u - (uint32_t)__clzll((long long)m0)) * st;
-      const uint32_t b1 = (63u - (uint32_t)__clzll((long long)m1)) * st;
-      const uint64_t n0 = __ballot(lane < st && sm.woff[min(b0 + lane, v.n_par)] <= w0);
-      const uint64_t n1 = __ballot(lane < st && sm.woff[min(b1 + lane, v.n_par)] <= wl);
-      pa = b0 + (63u - (uint32_t)__clzll((long long)n0));
-      pb = b1 + (63u - (uint32_t)__clzll((long long)n1)) + 1u;
-    }
-    if (w < W) {
-      // parent of work item w: the last j with woff[j] <= w
-      uint32_t lo = pa, hi = pb;
-      if (v.one_each) {
-        lo = w;
-      } else {
-        while (hi - lo > 1) {
-          const uint32_t mid = (lo + hi) >> 1;
-          const uint32_t o = lds_par ? sm.woff[mid] : ld_relaxed(&v.woff[mid]);
-          if (o <= w) lo = mid; else hi = mid;
+    // the item of this lane: its parent and its place among the parent's
+    bool item_ok;
+    uint32_t q = 0;
+    bool matched = false;  // (queued) its first fingerprint word matched
+    if (queued) {
+      while (n_q < 64u && c < nchunks) {
+        // what each item is (pk) and the word its filter looks at (every lane
+        // reads, an item without a filter the first label, so that the reads
+        // of all the chunks go out before the first is waited for)
+        uint32_t pk[kQueueChunks];
+        uint64_t pw[kQueueChunks];
+#pragma unroll
+        for (uint32_t u = 0; u < kQueueChunks; ++u) {
+          pk[u] = kPkNone;
+          const uint64_t* at = (const uint64_t*)labels;
+          const uint32_t w = (c << 6) + lane;
+          if (c < nchunks) {
+            // the chunk's parents: at or after the last chunk's, in one round
+            // of the search above when they are among the next 64
+            const uint32_t w0 = c << 6, wl = min(w0 + 63u, W - 1u);
+            const uint32_t o = sm.woff[min(p_at + lane, v.n_par)];
+            const uint64_t m0 = __ballot(o <= w0), m1 = __ballot(o <= wl);
+            uint32_t pa = p_at + (63u - (uint32_t)__clzll((long long)m0));
+            uint32_t pb = p_at + (64u - (uint32_t)__clzll((long long)m1));
+            if (m1 == ~0ull) chunk_parents(c, pa, pb);
+            p_at = pa;
+            if (w < W) {
+              uint32_t lo = pa, hi = pb;
+              while (hi - lo > 1) {
+                const uint32_t mid = (lo + hi) >> 1;
+                if (sm.woff[mid] <= w) lo = mid; else hi = mid;
+              }
+              const uint32_t i = w - sm.woff[lo], md = sm.p_mode[lo], c0 = sm.p_c0[lo];
+              const uint32_t item = (lo << 16) | i;
+              pk[u] = kPkAll | item;
+              if ((md & kModeMask) == M_SCAN) {
+                const uint32_t n = c0 + i;
+                ++my_children;
+                pk[u] = kPkScan | item | ((n & 1u) ? kPkBit : 0u);
+                at = (const uint64_t*)(labels + (n & ~1u));
+              } else if ((md & kModeMask) == M_HASH) {
+                const double x = (double)sm.row_lp[i], s = sm.p_s[lo] + x;
+                bool low = x <= (double)v.tok_thr || s <= v.sent_thr;
+                // a proposal on the round's other side of the cut is not
+                // looked up where its child could only go to `next`
+                if (v.cut_mode != kCutNone && ((md & kModeOpen) || !(md & kModeDepthOk) ||
+                                               v.cut_mode == kCutBelow))
+                  low = low || (s * v.lnf_next >= v.cut) != (v.cut_mode == kCutAbove);
+                if (low) {
+                  pk[u] = kPkNone;
+                } else if (md & kModeFiltered) {
+                  pk[u] = kPkHash | item;
+                  at = wfp + (c0 + cuckoo_h1(sm.row_id[i], sm.p_aux[lo]));
+                }
+              }
+            }
+          }
+          c += nwaves;
+          pw[u] = *at;
+        }
+#pragma unroll
+        for (uint32_t u = 0; u < kQueueChunks; ++u) {
+          const uint32_t kind = pk[u] & kPkNone;
+          const uint32_t w0 = (uint32_t)pw[u], w1 = (uint32_t)(pw[u] >> 32);
+          bool want = kind == kPkAll;
+          uint32_t e = pk[u];
+          if (kind == kPkScan) {
+            const uint32_t bit = row_bit(((e & kPkBit) ? w1 : w0) & kTokMask);
+            want = (sm.rh_bits[bit >> 5] >> (bit & 31u)) & 1u;
+          } else if (kind == kPkHash) {
+            const uint32_t f4 = wide_fp(sm.row_id[e & 0xFFFFu]) * 0x01010101u;
+            const bool first = has_zero_byte(w0 ^ f4) || has_zero_byte(w1 ^ f4);
+            // (a full first bucket without a match: the second may hold it)
+            want = first || !(has_zero_byte(w0) || has_zero_byte(w1));
+            if (first) e |= kPkBit;
+          }
+          const uint64_t m = __ballot(want);
+          if (want) qd[n_q + lanemask_lt_count(m)] = e;
+          n_q += (uint32_t)__popcll(m);
         }
       }
-      pj = lo;
-      uint32_t md, c0, aux, q;
+      if (n_q == 0) break;
+      // (the queue is the wave's own: LDS runs a wave's accesses in order)
+      __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+      const uint32_t take = min(n_q, 64u);
+      n_q -= take;
+      item_ok = lane < take;
+      if (item_ok) {
+        const uint32_t e = qd[n_q + lane];
+        pj = (e & kPkItem) >> 16;
+        q = e & 0xFFFFu;
+        matched = (e & kPkBit) != 0;
+      }
+      __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    } else {
+      if (c >= nchunks) break;
+      const uint32_t w = (c << 6) + lane;
+      uint32_t pa = 0, pb = v.n_par;
+      if (lds_par && !v.one_each) chunk_parents(c, pa, pb);
+      c += nwaves;
+      item_ok = w < W;
+      if (item_ok) {
+        // parent of work item w: the last j with woff[j] <= w
+        uint32_t lo = pa, hi = pb;
+        if (v.one_each) {
+          lo = w;
+        } else {
+          while (hi - lo > 1) {
+            const uint32_t mid = (lo + hi) >> 1;
+            const uint32_t o = lds_par ? sm.woff[mid] : ld_relaxed(&v.woff[mid]);
+            if (o <= w) lo = mid; else hi = mid;
+          }
+        }
+        pj = lo;
+        q = w - (lds_par ? sm.woff[pj] : ld_relaxed(&v.woff[pj]));
+      }
+    }
+    if (item_ok) {
+      uint32_t md, c0, aux;
       if (lds_par) {
-        q = w - sm.woff[pj];
         md = sm.p_mode[pj];
         c0 = sm.p_c0[pj];
         aux = sm.p_aux[pj];
       } else {
-        q = w - ld_relaxed(&v.woff[pj]);
         md = ld_relaxed(&v.pmode[pj]);
         c0 = ld_relaxed(&v.pc0[pj]);
         aux = ld_relaxed(&v.paux[pj]);
@@ -1161,7 +1411,7 @@ __device__ __forceinline__ void expand_range(const KArgs& a, const StepView& v, 
         // the child's label: its first token, and whether it closes a key
         cnode = c0 + q;
         const uint32_t lw = a.labels[cnode];
-        ++my_children;
+        if (!queued) ++my_children;
         ftok = lw & kTokMask;
         have_child = true;
         label_sel = (lw & kSlotSel) && depth_ok;
@@ -1169,11 +1419,11 @@ __device__ __forceinline__ void expand_range(const KArgs& a, const StepView& v, 
         pos = (int)q;
       }
       if (ftok != kNoToken)
-        pos = K > kMaxLdsTopk ? grow_find((const uint32_t*)sm.grow_id, K, ftok)
+        pos = !kLean && K > kMaxLdsTopk ? grow_find((const uint32_t*)sm.grow_id, K, ftok)
                               : row_find(sm, K, ftok, hashed);
       if (pos >= 0) {
         float x;
-        if (K > kMaxLdsTopk) {
+        if (!kLean && K > kMaxLdsTopk) {
           x = __uint_as_float(ld_relaxed((const uint32_t*)sm.grow_lp + pos));
           tok = ld_relaxed((const uint32_t*)sm.grow_id + pos);
         } else {
@@ -1214,7 +1464,7 @@ __device__ __forceinline__ void expand_range(const KArgs& a, const StepView& v, 
             // a filtered table: no fingerprint match in the first bucket
             // (nor in the second, when the first is full) means no child
             bool maybe = true;
-            if (filtered) {
+            if (filtered && !matched) {
               const uint64_t f8 = (uint64_t)wide_fp(tok) * 0x0101010101010101ull;
               const uint64_t w1 = a.wfp[b];
               maybe = has_zero_byte(w1 ^ f8);
@@ -1267,6 +1517,11 @@ __device__ __forceinline__ void expand_range(const KArgs& a, const StepView& v, 
             // length t + 1 (louds-trie.cc:103-108)
             do_next = true;
             do_sel = label_sel;
+          }
+          if (kLean && v.cut_mode != kCutNone) {
+            const bool above = s2 * v.lnf_next >= v.cut;
+            do_next = do_next && above == (v.cut_mode == kCutAbove);
+            do_sel = do_sel && v.cut_mode == kCutAbove;
           }
         }
       }
@@ -1364,12 +1619,21 @@ __device__ __forceinline__ void load_row(const uint32_t* rid, const float* rlp, 
 // token and are left out.  Row tokens are distinct (staging rejects
 // duplicates) and fill at most half the table (K <= kRowHashMaxK), so every
 // insert ends in a free slot.
+// kBits: the row's token bits (kRowBits) too, which the queued steps look at.
+template <bool kBits>
 __device__ __forceinline__ void row_hash_clear(Smem& sm) {
   for (uint32_t i = threadIdx.x; i < (uint32_t)kRowHash; i += kBlock)
     sm.rh_tok[i] = kRowHashEmpty;
+  if constexpr (kBits)
+    for (uint32_t i = threadIdx.x; i < kRowBits / 32u; i += kBlock) sm.rh_bits[i] = 0u;
 }
+template <bool kBits>
 __device__ __forceinline__ void row_hash_insert(uint32_t tok, uint32_t p, Smem& sm) {
   if (tok >= kTokMask) return;
+  if constexpr (kBits) {
+    const uint32_t bit = row_bit(tok);
+    atomicOr(&sm.rh_bits[bit >> 5], 1u << (bit & 31u));
+  }
   uint32_t h = row_hash(tok);
   for (int it = 0; it < kRowHash; ++it) {
     if (atomicCAS(&sm.rh_tok[h], kRowHashEmpty, tok) == kRowHashEmpty) {
@@ -1382,10 +1646,11 @@ __device__ __forceinline__ void row_hash_insert(uint32_t tok, uint32_t p, Smem& 
 
 // Hashes the LDS row (the workgroup has synchronised since the row was
 // written).  Ends synchronised.
+template <bool kBits>
 __device__ __forceinline__ void hash_row(uint32_t K, Smem& sm) {
-  row_hash_clear(sm);
+  row_hash_clear<kBits>(sm);
   __syncthreads();
-  for (uint32_t p = threadIdx.x; p < K; p += kBlock) row_hash_insert(sm.row_id[p], p, sm);
+  for (uint32_t p = threadIdx.x; p < K; p += kBlock) row_hash_insert<kBits>(sm.row_id[p], p, sm);
   __syncthreads();
 }
 
@@ -1661,7 +1926,7 @@ __device__ __forceinline__ bool ensure_rows(const KArgs& a, uint32_t req, const 
 
 // A helper workgroup: waits for shared steps of its request and expands its
 // slice of the work items, until the leader posts the exit generation.
-template <bool kStreamed>
+template <bool kStreamed, bool kLean>
 __device__ __forceinline__ void helper_loop(const KArgs& a, const DevReq& d, uint8_t* ws,
                             uint32_t g, Smem& sm) {
   const uint32_t tid = threadIdx.x;
@@ -1724,7 +1989,7 @@ __device__ __forceinline__ void helper_loop(const KArgs& a, const DevReq& d, uin
       if (acc == 0x9E3779B9u) sm.w_probes = acc;
     }
   }
-  row_hash_clear(sm);  // (visible after the first barrier below)
+  row_hash_clear<kLean>(sm);  // (visible after the first barrier below)
   for (;;) {
     if (tid == 0) {
       unsigned long long v = 0;
@@ -1752,6 +2017,8 @@ __device__ __forceinline__ void helper_loop(const KArgs& a, const DevReq& d, uin
         sm.hstep[1] = pW;
         sm.hstep[2] = pn;
         sm.hstep[3] = pS;
+        sm.hcut = ld_relaxed(&ctl->cut);
+        sm.hcut_mode = ld_relaxed(&ctl->cut_mode);
         sm.hstep[4] = ld_relaxed(&ctl->cur_which);
         sm.hstep[5] = ld_relaxed(&ctl->sel_which);
         // A posted step always satisfies the bounds below; a claimed slice
@@ -1766,7 +2033,8 @@ __device__ __forceinline__ void helper_loop(const KArgs& a, const DevReq& d, uin
     const unsigned long long v = sm.bcast;
     const uint32_t t = sm.hstep[0], W = sm.hstep[1], n_par = sm.hstep[2],
                    nS = sm.hstep[3], cur_which = sm.hstep[4], sel_which = sm.hstep[5];
-    const uint32_t mine = sm.hstep[6];
+    const uint32_t mine = sm.hstep[6], cut_mode = sm.hcut_mode;
+    const double cut = __longlong_as_double((long long)sm.hcut);
     __syncthreads();
     if ((v >> 32) != a.epoch || (uint32_t)v == kGoExit || v == seen) return;
     seen = v;
@@ -1808,13 +2076,15 @@ __device__ __forceinline__ void helper_loop(const KArgs& a, const DevReq& d, uin
     sv.sent_thr = d.sent_thr;
     sv.keep_lds_max = 0;
     sv.one_each = false;
+    sv.cut = cut;
+    sv.cut_mode = cut_mode;
     // the step's row (into the row hash too: emptied after the previous
     // step) and parent table in one round of reads; a row longer than the
     // LDS row arrays is searched where it is staged
-    const bool hashed = d.K <= kRowHashMaxK;
-    const bool lds_par = n_par <= (uint32_t)kBlock;
+    const bool hashed = kLean || d.K <= kRowHashMaxK;
+    const bool lds_par = kLean || n_par <= (uint32_t)kBlock;
     const uint64_t ro = (uint64_t)t * d.K;
-    const bool big = d.K > kMaxLdsTopk;
+    const bool big = !kLean && d.K > kMaxLdsTopk;
     if (big && tid == 0) {
       sm.grow_id = (unsigned long long)(rid + ro);
       sm.grow_lp = (unsigned long long)(rlp + ro);
@@ -1848,7 +2118,7 @@ __device__ __forceinline__ void helper_loop(const KArgs& a, const DevReq& d, uin
       if (i < Kl) {
         sm.row_id[i] = tok;
         sm.row_lp[i] = lp;
-        if (hashed) row_hash_insert(tok, i, sm);
+        if (hashed) row_hash_insert<kLean>(tok, i, sm);
       }
     }
     if (tid == 0) {
@@ -1858,10 +2128,10 @@ __device__ __forceinline__ void helper_loop(const KArgs& a, const DevReq& d, uin
       sm.lq_sel = 0;
     }
     __syncthreads();
-    expand_range(a, sv, W, g * (uint32_t)kWaves, a.wgs * (uint32_t)kWaves, false, false,
-                 hashed, sm);
+    expand_range<kLean>(a, sv, W, g * (uint32_t)kWaves, a.wgs * (uint32_t)kWaves, false, false,
+                        hashed, sm);
     // the row lookups are done: empty the hash for the next step
-    if (hashed) row_hash_clear(sm);
+    if (hashed) row_hash_clear<kLean>(sm);
     if (tid == 0) st_dev(dw + 1, pack2(sm.w_children, sm.w_probes));
     wait_stores();  // this slice's pushes and counters are complete
     __syncthreads();
@@ -2165,7 +2435,7 @@ __device__ __forceinline__ void tiny_steps(
     hist_used += n_next;
     nS += n_new;
     cands += (uint64_t)n_next + n_new;
-    if (lane == 0) sm.cnt_parents += n_cur;
+    if (lane == 0) lds_add(&sm.cnt_parents, n_cur);
     n_cur = n_next;
     ticks += c1 - c0;
     c0 = c1;
@@ -2217,7 +2487,14 @@ __device__ __forceinline__ void tiny_steps(
 // friends).  Separate instantiations, so that each keeps its own register
 // allocation and code: the staged search carries none of the streamed
 // one's start and output.
-template <bool kLouds, bool kStreamed>
+// kLean: every beam and row of the launch is at most kBlock long (launch_tbs
+// is told), so that the parent table and the row of a step are always in LDS,
+// one thread an entry.  The instantiation leaves out the code for longer ones
+// and queues the items of large steps: 100 KB of code against 117 KB with
+// neither, which pays at every step since the leader's loop does not fit the
+// 64 KB instruction cache (the queue beside the general code made calls of
+// batch 1 3-5% slower).
+template <bool kLouds, bool kStreamed, bool kLean>
 __global__ void __launch_bounds__(kBlock) tbs_kernel(KArgs a) {
   __shared__ Smem sm;
   // request-major interleave: request r owns blocks r, r + batch, ...  The
@@ -2242,7 +2519,7 @@ __global__ void __launch_bounds__(kBlock) tbs_kernel(KArgs a) {
     return;
   }
   if (g != 0) {
-    helper_loop<kStreamed>(a, d, ws, g, sm);
+    helper_loop<kStreamed, kLean>(a, d, ws, g, sm);
     return;
   }
 
@@ -2297,9 +2574,8 @@ __global__ void __launch_bounds__(kBlock) tbs_kernel(KArgs a) {
                  hist_cap = a.lay.hist_cap;
   const unsigned long long tag = (unsigned long long)a.epoch << 32;
   uint32_t gen = 0;
-  unsigned long long t_post = 0;  // (thread 0) wall clock of the last post
 
-  unsigned long long t_exp = 0, t_sel = 0, t_all0 = wall_clock64();
+  if (tid == 0) sm.t_all0 = wall_clock64();
   // per-step profile rows after the output tokens: kStepStats u64 per step
   uint64_t* step_stats = (uint64_t*)(ob + step_stats_offset(d.F, d.out_T));
   for (uint32_t i = tid; i < d.out_T * kStepStats; i += kBlock) step_stats[i] = 0;
@@ -2308,14 +2584,14 @@ __global__ void __launch_bounds__(kBlock) tbs_kernel(KArgs a) {
     sm.status = 0;
     sm.multi_item = 0;
     sm.cnt_parents = sm.cnt_children = sm.cnt_probes = 0;
+    sm.t_exp = sm.t_sel = sm.n_cands = 0;
   }
   uint32_t n_cur = 1, nS = 0, hist_used = 0;
-  uint64_t n_cands = 0;
   // the parent table of the step was written by the previous step's emit,
   // and its row loaded into registers there (pf_*); for step 0 both are
   // read here, the root's entry by one thread of wave 1 while every thread
   // reads its share of row 0
-  bool par_ready = true, row_pf = K <= (uint32_t)kBlock;
+  bool par_ready = true, row_pf = kLean || K <= (uint32_t)kBlock;
   uint32_t pf_id = 0;
   float pf_lp = 0.0f;
   if (row_pf && tid < K) {
@@ -2366,7 +2642,7 @@ __global__ void __launch_bounds__(kBlock) tbs_kernel(KArgs a) {
     // (no bounded selection cuts and early exit does not fire mid-step); at
     // the first step that needs a cut it hands the beam back to the general
     // step.
-    if (par_ready && n_cur <= 64u && K <= (uint32_t)kBlock) {
+    if ((kLean || (par_ready && K <= (uint32_t)kBlock)) && n_cur <= 64u) {
       const uint32_t lane = tid & 63u;
       const uint32_t md0 = lane < n_cur ? (uint32_t)(sm.p_mode[lane] & kModeMask) : (uint32_t)M_LP_NEXT;
       if (__ballot(md0 != M_LP_NEXT && md0 != M_LP_SEL) == 0) {
@@ -2390,8 +2666,10 @@ __global__ void __launch_bounds__(kBlock) tbs_kernel(KArgs a) {
           n_cur = sm.tiny_ncur;
           nS = sm.tiny_nS;
           hist_used = sm.tiny_hist;
-          n_cands += sm.tiny_cands;
-          t_exp += sm.tiny_ticks;
+          if (tid == 0) {
+            lds_add(&sm.n_cands, sm.tiny_cands);
+            lds_add(&sm.t_exp, sm.tiny_ticks);
+          }
           if (sm.tiny_done || sm.status) {
             finished = true;
             break;
@@ -2416,7 +2694,7 @@ __global__ void __launch_bounds__(kBlock) tbs_kernel(KArgs a) {
         sm.row_lp[tid] = pf_lp;
       }
     } else {
-      if (K <= kMaxLdsTopk) {
+      if (kLean || K <= kMaxLdsTopk) {
         load_row(rid, rlp, t, K, sm);
       } else if (tid == 0) {
         // a row longer than the LDS row arrays is searched in the stage
@@ -2434,8 +2712,8 @@ __global__ void __launch_bounds__(kBlock) tbs_kernel(KArgs a) {
       // (an opaque index: the per-thread addresses below are formed here,
       // not hoisted out of the step loop into registers held all along)
       asm volatile("" : "+v"(j));
-      const bool lp = n_cur <= (uint32_t)kBlock;
-      if (par_ready) {
+      const bool lp = kLean || n_cur <= (uint32_t)kBlock;
+      if (kLean || par_ready) {
         if (lp) {
           const uint32_t md = sm.p_mode[j], c0 = sm.p_c0[j], cur_lp = sm.p_lp[j];
           sm.x_s[j] = sm.p_s[j];
@@ -2493,25 +2771,25 @@ __global__ void __launch_bounds__(kBlock) tbs_kernel(KArgs a) {
         }
       }
     } else {
-      for (uint32_t cbase = 0; cbase < n_cur; cbase += kBlock) {
+      for (uint32_t cbase = 0; cbase < (kLean ? 1u : n_cur); cbase += kBlock) {
         const uint32_t j = cbase + tid;
         const uint32_t work = j < n_cur ? parent_work(j) : 0u;
         uint32_t Wc;
         const uint32_t off = block_excl_scan(work, &Wc, sm);
         if (j < n_cur) {
           st_dev(&par_woff[j], W + off);
-          if (n_cur <= (uint32_t)kBlock) sm.woff[j] = W + off;
+          if (kLean || n_cur <= (uint32_t)kBlock) sm.woff[j] = W + off;
           if (work != 1) sm.multi_item = 1;
         }
         W += Wc;
       }
       if (tid == 0) {
         st_dev(&par_woff[n_cur], W);
-        if (n_cur <= (uint32_t)kBlock) sm.woff[n_cur] = W;
+        if (kLean || n_cur <= (uint32_t)kBlock) sm.woff[n_cur] = W;
       }
     }
     if (tid == 0) {
-      sm.cnt_parents += n_cur;
+      lds_add(&sm.cnt_parents, n_cur);
       // this workgroup's expansion counters (expand_range of the leader
       // relies on them being zero)
       sm.w_children = 0;
@@ -2542,93 +2820,109 @@ __global__ void __launch_bounds__(kBlock) tbs_kernel(KArgs a) {
     sv.tok_thr = d.tok_thr;
     sv.sent_thr = d.sent_thr;
     sv.keep_lds_max = min((uint32_t)kPushCap, beams[t]);
-    sv.one_each = n_cur <= (uint32_t)kBlock && sm.multi_item == 0;
+    sv.one_each = (kLean || n_cur <= (uint32_t)kBlock) && sm.multi_item == 0;
 
 
     const bool shared = a.wgs > 1 && W >= a.share_min;
-    if (shared) {
-      // publish the step (the helpers read the row from the staged request),
-      // then wake the helpers
-      if (tid == 0) {
-        st_dev(&ctl->pushes, 0ull);
-        st_dev(&ctl->t, t);
-        st_dev(&ctl->W, W);
-        st_dev(&ctl->n_par, n_cur);
-        st_dev(&ctl->nS, nS);
-        st_dev(&ctl->sel_which, sel_which);
-        st_dev(&ctl->cur_which, cur_which);
-        st_dev(&ctl->hist_n, hist_used);
+    sv.cut = 0.0;
+    sv.cut_mode = kCutNone;
+    const bool hashed = (kLean || K <= kRowHashMaxK) && W >= kRowHashMinWork;
+    if (kLean && shared && queues_items(a, sv, W, a.wgs * (uint32_t)kWaves, hashed))
+      cut_of_step(a, sv, beams[t], (const uint64_t*)(in + d.kb_off) + 2ull * t, sm);
+    // the leader's slice 0, then (shared) the slices it takes over: one call
+    // of the inlined expansion for both, which keeps its code and registers
+    // to one copy
+    uint32_t sh_next = 0, sh_sel = 0;  // (shared) the pushes of the step
+    uint32_t lead_ch = 0, lead_pr = 0;  // the counters of the leader's slices
+    uint32_t n_stolen = 0;
+    bool stole = false;  // (thread i) slice i + 1 was taken over here
+    const uint32_t nh = a.wgs - 1;  // helper slots 1 .. nh (nh < kBlock)
+    // one round, or two when a cut let too few pushes through
+    for (;;) {
+      if (shared) {
+        // publish the step (the helpers read the row from the staged request),
+        // then wake the helpers
+        if (tid == 0) {
+          if (sv.cut_mode != kCutBelow) st_dev(&ctl->pushes, 0ull);
+          st_dev(&ctl->t, t);
+          st_dev(&ctl->W, W);
+          st_dev(&ctl->n_par, n_cur);
+          st_dev(&ctl->nS, nS);
+          st_dev(&ctl->sel_which, sel_which);
+          st_dev(&ctl->cur_which, cur_which);
+          st_dev(&ctl->hist_n, hist_used);
+          st_dev(&ctl->cut, (unsigned long long)__double_as_longlong(sv.cut));
+          st_dev(&ctl->cut_mode, sv.cut_mode);
+        }
+        wait_stores();  // the step's data is complete before `go` moves
+        __syncthreads();
+        ++gen;
+        if (tid == 0) {
+          st_dev(&ctl->go, tag | gen);
+          sm.t_post = wall_clock64();
+        }
       }
-      wait_stores();  // the step's data is complete before `go` moves
-      __syncthreads();
-      ++gen;
-      if (tid == 0) {
-        st_dev(&ctl->go, tag | gen);
-        t_post = wall_clock64();
+      // (the parent table ended synchronised: the row and the emptied hash are
+      // visible)
+      if (hashed && sv.cut_mode != kCutBelow) hash_row<kLean>(K, sm);
+      // (streamed) helper 1 copying the request's later rows claims no slice
+      // meanwhile: its slice is taken over at once rather than after the
+      // grace period (thread 0 stands for slot 1 below)
+      bool copying1 = false;
+      if constexpr (kStreamed) {
+        if (shared && tid == 0 && !ss.done && !ss.own && ss.split < T)
+          copying1 = ld_relaxed(&ctl->copy) == (tag | kCopyClaimed);
       }
-    }
-    // (the parent table ended synchronised: the row and the emptied hash are
-    // visible)
-    const bool hashed = K <= kRowHashMaxK && W >= kRowHashMinWork;
-    if (hashed) hash_row(K, sm);
-    // (streamed) helper 1 copying the request's later rows claims no slice
-    // meanwhile: its slice is taken over at once rather than after the
-    // grace period (thread 0 stands for slot 1 below)
-    bool copying1 = false;
-    if constexpr (kStreamed) {
-      if (shared && tid == 0 && !ss.done && !ss.own && ss.split < T)
-        copying1 = ld_relaxed(&ctl->copy) == (tag | kCopyClaimed);
-    }
-    expand_range(a, sv, W, 0, (shared ? a.wgs : 1u) * (uint32_t)kWaves, true, !shared,
-                 hashed, sm);
-    // (shared) the pushes of the step; the counters of the leader's slices
-    uint32_t sh_next = 0, sh_sel = 0, lead_ch = sm.w_children, lead_pr = sm.w_probes;
-    if (shared) {
-      // The helpers' slices: each is claimed by its helper (its claim word
-      // set to this step) or, once kGraceTicks have passed since the post,
-      // taken over here -- so the step never waits for a workgroup that is
-      // not running.  Then every claimed slice is waited for: a helper that
-      // claimed one is running and finishes it.
-      const unsigned long long tw0 = wall_clock64();
       const unsigned long long mygo = tag | gen;
-      unsigned long long* claims = (unsigned long long*)(ws + a.lay.claims);
-      const uint32_t nh = a.wgs - 1;  // helper slots 1 .. nh (nh < kBlock)
-      bool pending_any = true;
-      for (;;) {
-        const int pending = __syncthreads_count(tid < nh && !copying1 &&
-                                                ld_relaxed(&claims[tid + 1]) != mygo);
-        if (pending == 0) {
-          pending_any = false;
-          break;
+      for (uint32_t taken = 0, slice = 0;;) {
+        expand_range<kLean>(a, sv, W, slice * (uint32_t)kWaves,
+                            (shared ? a.wgs : 1u) * (uint32_t)kWaves, true, !shared, hashed, sm);
+        lead_ch += sm.w_children;
+        lead_pr += sm.w_probes;
+        if (!shared) break;
+        if (slice == 0) {
+          // The helpers' slices: each is claimed by its helper (its claim word
+          // set to this step) or, once kGraceTicks have passed since the post,
+          // taken over here -- so the step never waits for a workgroup that is
+          // not running.  Then every claimed slice is waited for: a helper that
+          // claimed one is running and finishes it.
+          if (tid == 0) sm.t_wait = wall_clock64();
+          unsigned long long* claims = (unsigned long long*)(ws + a.lay.claims);
+          bool pending_any = true;
+          for (;;) {
+            const int pending = __syncthreads_count(tid < nh && !copying1 &&
+                                                    ld_relaxed(&claims[tid + 1]) != mygo);
+            if (pending == 0) {
+              pending_any = false;
+              break;
+            }
+            if (tid == 0) sm.lead_flag = (wall_clock64() - sm.t_post > kGraceTicks) ? 1u : 0u;
+            __syncthreads();
+            const bool expired = sm.lead_flag != 0;
+            __syncthreads();
+            if (expired) break;
+            __builtin_amdgcn_s_sleep(2);
+          }
+          // (thread 0 alone knows whether helper 1 is copying: the takeover
+          // runs when any slot is still pending or helper 1 copies)
+          if (__syncthreads_or(pending_any || copying1)) {
+            if (tid == 0) sm.n_stolen = 0;
+            __syncthreads();
+            // raise every unclaimed word (helper 1's alone when only it is
+            // copying): a slice whose word this raises is taken over here; one
+            // a helper raised first stays the helper's
+            if (tid < nh && (pending_any || tid == 0) &&
+                atomicMax(&claims[tid + 1], mygo) < mygo) {
+              stole = true;
+              const uint32_t k = atomicAdd(&sm.n_stolen, 1u);
+              sm.stolen[k] = (uint16_t)(tid + 1);
+            }
+            __syncthreads();
+            n_stolen = sm.n_stolen;
+          }
         }
-        if (tid == 0) sm.lead_flag = (wall_clock64() - t_post > kGraceTicks) ? 1u : 0u;
-        __syncthreads();
-        const bool expired = sm.lead_flag != 0;
-        __syncthreads();
-        if (expired) break;
-        __builtin_amdgcn_s_sleep(2);
-      }
-      uint32_t n_stolen = 0;
-      bool stole = false;  // (thread i) slice i + 1 was taken over here
-      // (thread 0 alone knows whether helper 1 is copying: the takeover
-      // runs when any slot is still pending or helper 1 copies)
-      if (__syncthreads_or(pending_any || copying1)) {
-        if (tid == 0) sm.n_stolen = 0;
-        __syncthreads();
-        // raise every unclaimed word (helper 1's alone when only it is
-        // copying): a slice whose word this raises is taken over here; one
-        // a helper raised first stays the helper's
-        if (tid < nh && (pending_any || tid == 0) &&
-            atomicMax(&claims[tid + 1], mygo) < mygo) {
-          stole = true;
-          const uint32_t k = atomicAdd(&sm.n_stolen, 1u);
-          sm.stolen[k] = (uint16_t)(tid + 1);
-        }
-        __syncthreads();
-        n_stolen = sm.n_stolen;
-      }
-      for (uint32_t i = 0; i < n_stolen; ++i) {
-        const uint32_t slice = sm.stolen[i];
+        if (taken == n_stolen) break;
+        slice = sm.stolen[taken++];
         __syncthreads();
         if (tid == 0) {
           sm.w_children = 0;
@@ -2637,11 +2931,8 @@ __global__ void __launch_bounds__(kBlock) tbs_kernel(KArgs a) {
           sm.lq_sel = 0;
         }
         __syncthreads();
-        expand_range(a, sv, W, slice * (uint32_t)kWaves, a.wgs * (uint32_t)kWaves, true, false,
-                     hashed, sm);
-        lead_ch += sm.w_children;
-        lead_pr += sm.w_probes;
       }
+      if (!shared) break;
       // Every slice a helper claimed: thread i waits for helper i + 1's done
       // word to carry this step's tag (written after its pushes and its
       // counters are complete), unless thread i took that slice over.
@@ -2660,7 +2951,7 @@ __global__ void __launch_bounds__(kBlock) tbs_kernel(KArgs a) {
         if (!all_done) sm.status |= kStatusCorrupt;
         if (t < d.out_T) {
           uint64_t* row = step_stats + (uint64_t)t * kStepStats;
-          row[8] = tw1 - tw0;
+          row[8] = tw1 - sm.t_wait;
           row[9] = wall_clock64() - tw1;
         }
       }
@@ -2679,6 +2970,21 @@ __global__ void __launch_bounds__(kBlock) tbs_kernel(KArgs a) {
         if (wc) atomicAdd(&sm.w_children, wc);
         if (wp) atomicAdd(&sm.w_probes, wp);
       }
+      if (!kLean || sv.cut_mode != kCutAbove || sh_next >= beams[t] || !all_done) break;
+      // too few pushes reach the cut: the others, in a second round
+      sv.cut_mode = kCutBelow;
+      __syncthreads();
+      lead_ch = sm.w_children;
+      lead_pr = sm.w_probes;
+      n_stolen = 0;
+      stole = false;
+      __syncthreads();
+      if (tid == 0) {
+        sm.w_children = 0;
+        sm.w_probes = 0;
+        sm.lq_next = 0;
+        sm.lq_sel = 0;
+      }
     }
     __syncthreads();
     // the helpers' pushes are complete (they waited for their stores before
@@ -2692,10 +2998,10 @@ __global__ void __launch_bounds__(kBlock) tbs_kernel(KArgs a) {
     // 0 adds the overflow bit below, which every thread derives itself
     const bool overflow = n_next > next_cap || nS + n_new > sel_cap;
     const bool stop = overflow || sm.status != 0;
-    n_cands += (uint64_t)n_next + n_new;
     if (tid == 0) {
-      sm.cnt_children += w_ch;
-      sm.cnt_probes += w_pr;
+      lds_add(&sm.n_cands, (uint64_t)n_next + n_new);
+      lds_add(&sm.cnt_children, w_ch);
+      lds_add(&sm.cnt_probes, w_pr);
       if (overflow) sm.status |= kStatusOverflow;
     }
     if (stop) {
@@ -2703,7 +3009,7 @@ __global__ void __launch_bounds__(kBlock) tbs_kernel(KArgs a) {
       break;
     }
     const unsigned long long t1 = wall_clock64();
-    t_exp += t1 - t0;
+    if (tid == 0) lds_add(&sm.t_exp, t1 - t0);
     if (tid == 0 && t < d.out_T) {
       uint64_t* row = step_stats + (uint64_t)t * kStepStats;
       row[0] = ncur0;
@@ -2826,7 +3132,7 @@ __global__ void __launch_bounds__(kBlock) tbs_kernel(KArgs a) {
       }
     }
     if (stop_after) {
-      t_sel += wall_clock64() - t1;
+      if (tid == 0) lds_add(&sm.t_sel, wall_clock64() - t1);
       break;
     }
 
@@ -2838,7 +3144,7 @@ __global__ void __launch_bounds__(kBlock) tbs_kernel(KArgs a) {
       return rank[jk >> 16] * K + caller_index(rk, t, K, jk);
     };
     auto nn = [&](uint32_t i) { return nextc[i].node; };
-    const bool collect = M <= (uint32_t)kKeepCap;
+    const bool collect = kLean || M <= (uint32_t)kKeepCap;
     const uint64_t nk_lo = kbound[0], nk_hi = kbound[1];
     const Bound bn = bounded_select(n_next, M, nk, na, nn, compute_ranks, sm,
                                     nk_lo <= nk_hi, nk_lo, nk_hi, collect);
@@ -2866,7 +3172,7 @@ __global__ void __launch_bounds__(kBlock) tbs_kernel(KArgs a) {
     // survivor i becomes hypothesis o of the next beam
     // the next step's proposal row, into registers while the survivors are
     // emitted (the LDS row is still read until the emit ends)
-    row_pf = t + 1 < T && K <= (uint32_t)kBlock;
+    row_pf = t + 1 < T && (kLean || K <= (uint32_t)kBlock);
     if (row_pf && tid < K) {
       const uint64_t o = (uint64_t)(t + 1) * K + tid;
       pf_id = rid[o];
@@ -2877,12 +3183,12 @@ __global__ void __launch_bounds__(kBlock) tbs_kernel(KArgs a) {
     // with its table in place (in LDS as well when it has at most kBlock
     // parents).
     const bool next_table = t + 1 < T;
-    const bool next_lds = keep_cnt <= (uint32_t)kBlock;
+    const bool next_lds = kLean || keep_cnt <= (uint32_t)kBlock;
     // the parents' scores and history records, and their link tokens, are
     // in LDS when the step had at most kBlock parents; the row is, unless
     // the rank scratch took it
-    const bool x_ok = ncur_now <= (uint32_t)kBlock;
-    const bool row_ok = !ranks_done && K <= kMaxLdsTopk;
+    const bool x_ok = kLean || ncur_now <= (uint32_t)kBlock;
+    const bool row_ok = !ranks_done && (kLean || K <= kMaxLdsTopk);
     auto emit = [&](uint32_t i, uint32_t o) {
       const NextRec c = next_in_lds ? sm.push_next[i] : nextc[i];
       const uint32_t j = c.jk >> 16, q = c.jk & 0xFFFFu;
@@ -2981,7 +3287,7 @@ __global__ void __launch_bounds__(kBlock) tbs_kernel(KArgs a) {
       n_emit = min(sm.n_keep, (uint32_t)kKeepCap);
       from_list = true;
       if (tid == 0) sm.n_out = sm.n_keep;
-    } else if (keep_cnt <= (uint32_t)kKeepCap) {
+    } else if (kLean || keep_cnt <= (uint32_t)kKeepCap) {
       // positions of the survivors first (from the keys alone; the rest of
       // a record is read only for a key on the boundary of a cut tie)
       visit_keys(n_next, nk, [&](uint32_t i, bool ok, uint64_t key) {
@@ -2999,7 +3305,7 @@ __global__ void __launch_bounds__(kBlock) tbs_kernel(KArgs a) {
     } else {
       list_done = false;
     }
-    if (list_done) {
+    if (kLean || list_done) {
       // one dependent chain per survivor
       for (uint32_t o = tid; o < n_emit; o += kBlock)
         if (o < a.lay.cur_cap && hist_used + o < hist_cap)
@@ -3032,7 +3338,7 @@ __global__ void __launch_bounds__(kBlock) tbs_kernel(KArgs a) {
       cur_which ^= 1u;
     }
     par_ready = next_table;
-    t_sel += wall_clock64() - t1;
+    if (tid == 0) lds_add(&sm.t_sel, wall_clock64() - t1);
   }
   // release the helpers
   if (tid == 0) st_dev(&ctl->go, tag | kGoExit);
@@ -3149,10 +3455,10 @@ __global__ void __launch_bounds__(kBlock) tbs_kernel(KArgs a) {
   if (tid == 0) {
     oh->count = status ? 0 : nS;
     const unsigned long long tend = wall_clock64();
-    oh->ticks_expand = t_exp;
-    oh->ticks_select = t_sel;
-    oh->ticks_total = tend - t_all0;
-    oh->candidates = n_cands;
+    oh->ticks_expand = sm.t_exp;
+    oh->ticks_select = sm.t_sel;
+    oh->ticks_total = tend - sm.t_all0;
+    oh->candidates = sm.n_cands;
     oh->parents = sm.cnt_parents;
     oh->children = sm.cnt_children;
     oh->probes = sm.cnt_probes;
@@ -3234,14 +3540,22 @@ hipError_t launch_tbs(const KArgs& args, hipStream_t stream, hipEvent_t start,
   }
   if (args.louds_words) {
     if (args.ready) return hipErrorInvalidValue;  // (no streamed LOUDS search)
-    hipExtLaunchKernelGGL((tbs_kernel<true, false>), grid, block, 0, stream, start, stop, 0,
+    hipExtLaunchKernelGGL((tbs_kernel<true, false, false>), grid, block, 0, stream, start, stop, 0,
                           args);
   } else if (args.ready) {
-    hipExtLaunchKernelGGL((tbs_kernel<false, true>), grid, block, 0, stream, start, stop, 0,
-                          args);
+    if (args.lean)
+      hipExtLaunchKernelGGL((tbs_kernel<false, true, true>), grid, block, 0, stream, start, stop, 0,
+                            args);
+    else
+      hipExtLaunchKernelGGL((tbs_kernel<false, true, false>), grid, block, 0, stream, start, stop,
+                            0, args);
   } else {
-    hipExtLaunchKernelGGL((tbs_kernel<false, false>), grid, block, 0, stream, start, stop, 0,
-                          args);
+    if (args.lean)
+      hipExtLaunchKernelGGL((tbs_kernel<false, false, true>), grid, block, 0, stream, start, stop,
+                            0, args);
+    else
+      hipExtLaunchKernelGGL((tbs_kernel<false, false, false>), grid, block, 0, stream, start, stop,
+                            0, args);
   }
   return hipGetLastError();
 }
@@ -3265,7 +3579,8 @@ __global__ void __launch_bounds__(256) root_dir_kernel(KArgs a, RootEnt* dir, ui
   if ((r.meta & FT_META_TERMINAL) && el == 1u) f |= kRdSel;
   if (link) f |= kRdLink;
   if ((e.mode & kModeMask) == M_HASH)
-    f |= kRdTable | ((e.mode & kModeFiltered) ? kRdFiltered : 0u) | ((e.aux & 0xFFu) << 8);
+    f |= kRdTable | ((e.mode & kModeFiltered) ? kRdFiltered : 0u) |
+         ((e.mode & kModeOpen) ? kRdOpen : 0u) | ((e.aux & 0xFFu) << 8);
   if (err) f |= kRdErr;
   RootEnt o;
   o.node = ch;
@@ -3293,7 +3608,7 @@ int tbs_block_threads() { return kBlock; }
 
 int tbs_max_resident_blocks(int num_cus) {
   int per_cu = 0;
-  if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, (const void*)tbs_kernel<false, false>,
+  if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, (const void*)tbs_kernel<false, false, false>,
                                                    kBlock, 0) != hipSuccess)
     return 0;
   return per_cu * num_cus;
