@@ -255,6 +255,19 @@ __device__ __forceinline__ uint64_t norm_key(double v) {
 
 __device__ __forceinline__ uint32_t lane_id() { return threadIdx.x & 63; }
 
+// The thread's index; kHere: opaque, so that addresses formed from it are
+// formed where they are used.  The compiler otherwise forms the addresses of
+// loops inside the step loop in front of it and holds them in registers all
+// along -- in the lean instantiation more of them than fit, which took 20
+// bytes of scratch memory a lane (the runtime may have to allocate it at a
+// launch, which ft_search_noalloc promises not to cause).
+template <bool kHere>
+__device__ __forceinline__ uint32_t thread_idx() {
+  uint32_t t = threadIdx.x;
+  if constexpr (kHere) asm volatile("" : "+v"(t));
+  return t;
+}
+
 // whether some byte of v is zero
 __device__ __forceinline__ bool has_zero_byte(uint32_t v) {
   return ((v - 0x01010101u) & ~v & 0x80808080u) != 0;
@@ -466,18 +479,19 @@ __device__ __forceinline__ KeyT radix_kth(uint32_t n, uint32_t need, GetKey gk, 
 // thread (n >= 1 when the loop runs), with U items per thread in flight:
 // the reads are unconditional (a slot past the end re-reads item n - 1) so
 // that all of them are issued before the first is waited for.
-template <uint32_t U = 4, typename GetKey, typename F>
+template <bool kHere, uint32_t U = 4, typename GetKey, typename F>
 __device__ __forceinline__ void visit_keys(uint32_t n, GetKey gk, F f) {
+  const uint32_t tid = thread_idx<kHere>();
   for (uint32_t base = 0; base < n; base += U * kBlock) {
     uint64_t k[U];
 #pragma unroll
     for (uint32_t u = 0; u < U; ++u) {
-      const uint32_t i = base + u * kBlock + threadIdx.x;
+      const uint32_t i = base + u * kBlock + tid;
       k[u] = gk(min(i, n - 1u));
     }
 #pragma unroll
     for (uint32_t u = 0; u < U; ++u) {
-      const uint32_t i = base + u * kBlock + threadIdx.x;
+      const uint32_t i = base + u * kBlock + tid;
       f(i, i < n, k[u]);
     }
   }
@@ -495,18 +509,18 @@ __device__ __forceinline__ void visit_keys(uint32_t n, GetKey gk, F f) {
 // bins below the chosen one (sm.n_keep of them) and keeps the chosen bin's
 // positions in sm.bin_idx, and sm.collected says that it ran: then a bounded
 // selection needs no further pass over the list.
-template <typename GetKey>
+template <bool kHere, typename GetKey>
 __device__ __forceinline__ uint64_t kth_u64(uint32_t n, uint32_t need, GetKey gk, Smem& sm,
                             uint32_t* eq, uint32_t* rem_out, bool have_range,
                             uint64_t rmin, uint64_t rmax, bool collect = false) {
-  const uint32_t tid = threadIdx.x, lane = tid & 63u, wave = tid >> 6;
+  const uint32_t tid = thread_idx<kHere>(), lane = tid & 63u, wave = tid >> 6;
   if (tid == 0) sm.collected = 0;
   // key range: given (bounds of every key), or one pass
   uint64_t mn = rmin, mx = rmax;
   if (!have_range) {
     mn = ~0ull;
     mx = 0;
-    visit_keys(n, gk, [&](uint32_t, bool ok, uint64_t k) {
+    visit_keys<kHere>(n, gk, [&](uint32_t, bool ok, uint64_t k) {
       if (ok) {
         mn = min(mn, k);
         mx = max(mx, k);
@@ -552,7 +566,7 @@ __device__ __forceinline__ uint64_t kth_u64(uint32_t n, uint32_t need, GetKey gk
     const uint64_t hi_mask = (top >= 63) ? 0ull : ~((2ull << top) - 1ull);
     for (uint32_t i = tid; i < nb; i += kBlock) sm.whist[i] = 0;
     __syncthreads();
-    visit_keys<6>(n, gk, [&](uint32_t, bool ok, uint64_t k) {
+    visit_keys<kHere, 6>(n, gk, [&](uint32_t, bool ok, uint64_t k) {
       const uint64_t o = k - base;
       const bool act = ok && (o & hi_mask) == prefix;
       // (the wide bins spread a wave's keys: one LDS add a key, without
@@ -721,7 +735,7 @@ __device__ __forceinline__ bool bound_keep(const Bound& b, uint64_t key,
 // after `need_ranks()` has made parent ranks available.
 // With `have_range`, every key(i) lies in [kmin, kmax].  With `collect`,
 // see kth_u64 (the items with a key above the boundary bin are listed).
-template <typename GetKey, typename GetArr, typename GetNode, typename Ranks>
+template <bool kHere, typename GetKey, typename GetArr, typename GetNode, typename Ranks>
 __device__ __forceinline__ Bound bounded_select(uint32_t n, uint32_t M, GetKey key,
                                 GetArr arr, GetNode node, Ranks need_ranks,
                                 Smem& sm, bool have_range = false,
@@ -734,7 +748,7 @@ __device__ __forceinline__ Bound bounded_select(uint32_t n, uint32_t M, GetKey k
   }
   uint32_t eq, rem;
   // M-th largest key == M-th smallest of ~key
-  const uint64_t nk = kth_u64(n, M, [&](uint32_t i) { return ~key(i); }, sm, &eq,
+  const uint64_t nk = kth_u64<kHere>(n, M, [&](uint32_t i) { return ~key(i); }, sm, &eq,
                               &rem, have_range, ~kmax, ~kmin, collect);
   b.vkey = ~nk;
   if (eq == rem) return b;  // the whole boundary class fits
@@ -1151,7 +1165,7 @@ __device__ __forceinline__ bool queues_items(const KArgs& a, const StepView& v, 
 // 8, 510 -> 380 and 27.6 -> 18.1 us at batch 64.
 __device__ __forceinline__ void cut_of_step(const KArgs& a, StepView& v, uint32_t M,
                                             const uint64_t* kbound, Smem& sm) {
-  const uint32_t tid = threadIdx.x;
+  const uint32_t tid = thread_idx<true>();
   const uint64_t pairs = (uint64_t)v.n_par * v.K, want = (uint64_t)a.cut_pairs * M;
   const uint64_t klo = kbound[0], khi = kbound[1];
   if (want == 0 || 2 * want > pairs || klo >= khi) return;
@@ -1605,10 +1619,11 @@ __device__ __forceinline__ void expand_range(const KArgs& a, const StepView& v, 
 
 // Loads the proposal row of step t (staged in ascending token order) into
 // LDS.
+template <bool kHere>
 __device__ __forceinline__ void load_row(const uint32_t* rid, const float* rlp, uint32_t t,
                                          uint32_t K, Smem& sm) {
   const uint64_t o = (uint64_t)t * K;
-  for (uint32_t p = threadIdx.x; p < K; p += kBlock) {
+  for (uint32_t p = thread_idx<kHere>(); p < K; p += kBlock) {
     sm.row_id[p] = rid[o + p];
     sm.row_lp[p] = rlp[o + p];
   }
@@ -2540,8 +2555,9 @@ __global__ void __launch_bounds__(kBlock) tbs_kernel(KArgs a) {
   const uint8_t* in = a.stage + uni(d.in_off);
   const double* lnf = (const double*)in;
   const uint32_t* beams = (const uint32_t*)(in + d.beams_off);
-  const uint32_t* rid = (const uint32_t*)(in + d.rid_off);
-  const float* rlp = (const float*)(in + d.rlp_off);
+  // (the lean instantiation: in scalar registers, for want of others)
+  const uint32_t* rid = (const uint32_t*)(in + (kLean ? uni(d.rid_off) : d.rid_off));
+  const float* rlp = (const float*)(in + (kLean ? uni(d.rlp_off) : d.rlp_off));
   // the proposals' indices in the caller's rows, when some row came out of
   // order (else index = position)
   const uint16_t* rk = ss.rk ? (const uint16_t*)(in + d.rk_off) : nullptr;
@@ -2695,7 +2711,7 @@ __global__ void __launch_bounds__(kBlock) tbs_kernel(KArgs a) {
       }
     } else {
       if (kLean || K <= kMaxLdsTopk) {
-        load_row(rid, rlp, t, K, sm);
+        load_row<kLean>(rid, rlp, t, K, sm);
       } else if (tid == 0) {
         // a row longer than the LDS row arrays is searched in the stage
         // (the parent phase ends synchronised: every thread sees these)
@@ -2772,7 +2788,7 @@ __global__ void __launch_bounds__(kBlock) tbs_kernel(KArgs a) {
       }
     } else {
       for (uint32_t cbase = 0; cbase < (kLean ? 1u : n_cur); cbase += kBlock) {
-        const uint32_t j = cbase + tid;
+        const uint32_t j = cbase + (kLean ? thread_idx<kLean>() : tid);
         const uint32_t work = j < n_cur ? parent_work(j) : 0u;
         uint32_t Wc;
         const uint32_t off = block_excl_scan(work, &Wc, sm);
@@ -3095,7 +3111,7 @@ __global__ void __launch_bounds__(kBlock) tbs_kernel(KArgs a) {
           stop_after = true;
         }
       } else {
-        b = bounded_select(nU, F, sel_key, sel_arr, sel_node, compute_ranks, sm);
+        b = bounded_select<kLean>(nU, F, sel_key, sel_arr, sel_node, compute_ranks, sm);
       }
       if (b.all && !early_cut) {
         // every push fits: the new items simply become old ones (no LDS
@@ -3146,7 +3162,7 @@ __global__ void __launch_bounds__(kBlock) tbs_kernel(KArgs a) {
     auto nn = [&](uint32_t i) { return nextc[i].node; };
     const bool collect = kLean || M <= (uint32_t)kKeepCap;
     const uint64_t nk_lo = kbound[0], nk_hi = kbound[1];
-    const Bound bn = bounded_select(n_next, M, nk, na, nn, compute_ranks, sm,
+    const Bound bn = bounded_select<kLean>(n_next, M, nk, na, nn, compute_ranks, sm,
                                     nk_lo <= nk_hi, nk_lo, nk_hi, collect);
     // survivors already listed by the selection (keys above its boundary
     // bin), and the boundary bin's size
@@ -3290,7 +3306,7 @@ __global__ void __launch_bounds__(kBlock) tbs_kernel(KArgs a) {
     } else if (kLean || keep_cnt <= (uint32_t)kKeepCap) {
       // positions of the survivors first (from the keys alone; the rest of
       // a record is read only for a key on the boundary of a cut tie)
-      visit_keys(n_next, nk, [&](uint32_t i, bool ok, uint64_t key) {
+      visit_keys<kLean>(n_next, nk, [&](uint32_t i, bool ok, uint64_t key) {
         bool keep = false;
         if (ok) {
           if (bn.all || key > bn.vkey) keep = true;
