@@ -41,6 +41,7 @@
 #include <stdint.h>
 
 #include <mutex>
+#include <type_traits>
 
 #include "coherent.h"
 #include "tbs_kernel.h"
@@ -95,14 +96,9 @@ struct alignas(16) Smem {
   uint32_t n_next, n_sel, n_out, overflow;
   uint32_t status;
   unsigned long long cnt_parents, cnt_children, cnt_probes;
-  // thread 0's of the leader: its clocks and the candidates so far (here
-  // rather than in registers through the steps)
-  unsigned long long t_exp, t_sel, t_all0, t_post, t_wait, n_cands;
   unsigned long long bcast;
   uint32_t hstep[7];  // a helper's view of the posted step (+ whether it
                       // took its slice)
-  unsigned long long hcut;  // ... and its cut
-  uint32_t hcut_mode;
   uint32_t lead_flag;   // the leader's broadcast of a decision of thread 0
   uint32_t n_stolen;    // helper slices the leader took over this step
   uint16_t stolen[256];
@@ -136,8 +132,6 @@ struct alignas(16) Smem {
   uint8_t p_mode[kBlock];
   // link parents (kNoCursor otherwise): index in tail[] of the pending token
   uint32_t p_lp[kBlock];
-  // expansion: the row's token bits (see kRowBits)
-  uint32_t rh_bits[kRowBits / 32];
   // the leader's own per-parent data for its emit, which overwrites the
   // table above with the next step's, copied by the parent phase: score,
   // history record and, for a link parent that stays one on its own edge,
@@ -185,6 +179,20 @@ struct alignas(16) Smem {
   NextRec push_next[kPushCap];
   SelRec push_sel[kPushSelCap];
 };
+// What the lean instantiation (see tbs_kernel) holds besides, behind the
+// layout that both share.
+struct alignas(16) SmemLean : Smem {
+  // expansion: the row's token bits (see kRowBits)
+  uint32_t rh_bits[kRowBits / 32];
+  // a helper's view of the posted step's cut
+  unsigned long long hcut;
+  uint32_t hcut_mode;
+  // thread 0's of the leader: its clocks and the candidates so far (here
+  // rather than in registers through the steps)
+  unsigned long long t_exp, t_sel, t_all0, t_post, t_wait, n_cands;
+};
+template <bool kLean>
+using SmemOf = std::conditional_t<kLean, SmemLean, Smem>;
 // rank scratch aliases the row arrays (used after expansion only)
 constexpr int kRankChunk = 1024;
 static_assert(offsetof(Smem, row_id) % 16 == 0 && offsetof(Smem, row_lp) % 16 == 0,
@@ -859,7 +867,8 @@ constexpr uint32_t kNoToken = 0xFFFFFFFFu;
 struct ParEntry {
   uint32_t c0, aux, mode, work, lp;
 };
-template <bool kLouds>
+// kOpen: with kModeOpen, which the cuts of the lean instantiation look at.
+template <bool kLouds, bool kOpen>
 __device__ __forceinline__ ParEntry parent_entry(const KArgs& a, uint32_t node, uint32_t t,
                                                  uint32_t K, uint32_t* err) {
   // the node's home group in the table directory is read with its record
@@ -927,7 +936,7 @@ __device__ __forceinline__ ParEntry parent_entry(const KArgs& a, uint32_t node, 
           if (nds[k] == node) {
             found = true;
             e.mode = M_HASH | (((lgfs[k] >> 8) & kWideFiltered) ? kModeFiltered : 0u) |
-                     (((lgfs[k] >> 8) & kWideOpen) ? kModeOpen : 0u);
+                     (kOpen && ((lgfs[k] >> 8) & kWideOpen) ? kModeOpen : 0u);
             e.aux = lgfs[k] & 0xFFu;
             e.c0 = offs[k];
           }
@@ -947,6 +956,7 @@ __device__ __forceinline__ ParEntry parent_entry(const KArgs& a, uint32_t node, 
 // parent_entry(node, 1, K) of a root child from its root-directory entry
 // (x: node, flags, c0, deg; y: tab, link_tok, link_lp, sd): the same
 // branches, with the scan limit of this launch.
+template <bool kOpen>
 __device__ __forceinline__ ParEntry root_child_entry(const KArgs& a, const uint4 x,
                                                      const uint4 y, uint32_t K) {
   const uint32_t f = x.y, deg = x.w, sd = y.w;
@@ -967,7 +977,7 @@ __device__ __forceinline__ ParEntry root_child_entry(const KArgs& a, const uint4
     e.work = K;
     if (f & kRdTable) {
       e.mode = M_HASH | ((f & kRdFiltered) ? kModeFiltered : 0u) |
-               ((f & kRdOpen) ? kModeOpen : 0u);
+               (kOpen && (f & kRdOpen) ? kModeOpen : 0u);
       e.aux = (f >> 8) & 0xFFu;
       e.c0 = y.x;
     }
@@ -1208,6 +1218,172 @@ __device__ __forceinline__ void cut_of_step(const KArgs& a, StepView& v, uint32_
   v.cut_mode = kCutAbove;
 }
 
+// The child of a searched, hashed or dense parent (mode md, first child or
+// table c0, degree or table size aux) whose label is tok.  filtered: the
+// table's fingerprint words are looked at first.
+__device__ __forceinline__ void find_child(const KArgs& a, uint32_t md, uint32_t c0, uint32_t aux,
+                                           uint32_t tok, uint32_t t, bool depth_ok, bool filtered,
+                                           uint32_t& my_probes, uint32_t& cnode,
+                                           bool& have_child, bool& label_sel) {
+  if (md == M_SEARCH) {
+    // lower_bound of tok among the parent's children
+    uint32_t lo2 = c0, hi2 = c0 + aux;
+    const uint32_t end2 = hi2;
+    while (lo2 < hi2) {
+      const uint32_t mid = lo2 + ((hi2 - lo2) >> 1);
+      ++my_probes;
+      if (a.recs[mid].first_tok < tok) lo2 = mid + 1; else hi2 = mid;
+    }
+    if (lo2 < end2) {
+      const ft_node_rec cr = a.recs[lo2];
+      if (cr.first_tok == tok) {
+        cnode = lo2;
+        have_child = true;
+        // terminal with |KB| == |Q| -> selected (louds-trie.cc:103-108)
+        label_sel = (cr.meta & FT_META_TERMINAL) &&
+                    (cr.meta & FT_META_DEPTH_MASK) == t + 1;
+      }
+    }
+  } else if (md == M_HASH) {
+    // the token's first cuckoo bucket, and its second only when the
+    // first is full without a match
+    const uint32_t lg = aux;
+    uint32_t b = c0 + cuckoo_h1(tok, lg);
+    // a filtered table: no fingerprint match in the first bucket
+    // (nor in the second, when the first is full) means no child
+    bool maybe = true;
+    if (filtered) {
+      const uint64_t f8 = (uint64_t)wide_fp(tok) * 0x0101010101010101ull;
+      const uint64_t w1 = a.wfp[b];
+      maybe = has_zero_byte(w1 ^ f8);
+      if (!maybe && !has_zero_byte(w1))
+        maybe = has_zero_byte(a.wfp[c0 + cuckoo_h2(tok, lg)] ^ f8);
+    }
+    uint32_t hw = 0, hc = 0;
+    for (int round = 0; round < (maybe ? 2 : 0); ++round) {
+      // the whole bucket (tokens and children) in one read
+      const uint4* bw = (const uint4*)&a.wtab[b];
+      const uint4 ta = bw[0], tb = bw[1], ca = bw[2], cb = bw[3];
+      ++my_probes;
+      const uint32_t tw[8] = {ta.x, ta.y, ta.z, ta.w, tb.x, tb.y, tb.z, tb.w};
+      const uint32_t cw[8] = {ca.x, ca.y, ca.z, ca.w, cb.x, cb.y, cb.z, cb.w};
+      bool full = true;
+#pragma unroll
+      for (int sl = 0; sl < 8; ++sl) {
+        if ((tw[sl] & kTokMask) == tok) {
+          hw = tw[sl];
+          hc = cw[sl];
+        }
+        full = full && tw[sl] != kSlotEmptyTok;
+      }
+      if (hc != 0u || !full) break;
+      b = c0 + cuckoo_h2(tok, lg);
+    }
+    if (hc != 0u) {
+      cnode = hc;
+      have_child = true;
+      label_sel = (hw & kSlotSel) && depth_ok;
+    }
+  } else if (md == M_DENSE) {
+    // the root's child of this token: one read of (node, flags)
+    if (tok < a.root_n) {
+      const uint2 rd = *(const uint2*)&a.root_dir[tok];
+      ++my_probes;
+      if (rd.x != 0u) {
+        cnode = rd.x;
+        have_child = true;
+        label_sel = (rd.y & kRdSel) && depth_ok;
+      }
+    }
+  }
+}
+
+// Appends the lanes' pushes (every lane of the wave reaches these): into the
+// LDS buffers while they have room, the rest straight to the global lists.
+__device__ __forceinline__ void append_pushes(const StepView& v, bool do_next, bool do_sel,
+                                              double s2, uint32_t cnode, uint32_t pj, uint32_t k,
+                                              uint32_t tok, bool lds_par, bool solo, Smem& sm) {
+  const uint32_t t = v.t;
+  const uint32_t jk = (pj << 16) | k;
+  if (__ballot(do_next)) {
+    const uint32_t li = wave_append(do_next, &sm.lq_next);
+    const bool spill = do_next && li >= (uint32_t)kPushCap;
+    const uint32_t gi = solo ? li : wave_append_half(spill, &v.ctl->pushes, false);
+    if (do_next) {
+      const uint64_t key = norm_key(s2 * v.lnf_next);
+      if (!spill) {
+        sm.push_next[li].key = key;
+        sm.push_next[li].node = cnode;
+        sm.push_next[li].jk = jk;
+      } else if (gi < v.next_cap) {
+        st_next(&v.nextc[gi], key, cnode, jk);
+      }
+    }
+  }
+  if (__ballot(do_sel)) {
+    const uint32_t li = wave_append(do_sel, &sm.lq_sel);
+    const bool spill = do_sel && li >= (uint32_t)kPushSelCap;
+    const uint32_t gi = solo ? li : wave_append_half(spill, &v.ctl->pushes, true);
+    if (do_sel) {
+      SelRec sr;
+      sr.s = s2;
+      sr.node = cnode;
+      sr.depth = t + 1;
+      sr.phist = lds_par ? sm.p_hist[pj] : ld_cur(&v.cur[pj]).hist;
+      sr.tok = tok;
+      sr.jk = jk;
+      sr.isnew = 1;
+      if (!spill) sm.push_sel[li] = sr;
+      else if (v.nS + gi < v.sel_cap) st_sel(&v.sel[v.nS + gi], sr);
+    }
+  }
+}
+
+// The end of a workgroup's share of a step, once its items are expanded.
+__device__ __forceinline__ void expand_end(const StepView& v, uint32_t my_children,
+                                           uint32_t my_probes, bool solo, Smem& sm) {
+  const uint32_t tid = threadIdx.x;
+  // the workgroup's counters: one LDS add a wave (lane by lane, the adds to
+  // one word would run one after another, 1024 of them)
+  {
+    const uint32_t wc = wave_sum(my_children), wp = wave_sum(my_probes);
+    if ((tid & 63u) == 0u) {
+      if (wc) atomicAdd(&sm.w_children, wc);
+      if (wp) atomicAdd(&sm.w_probes, wp);
+    }
+  }
+  __syncthreads();
+  // the buffered pushes: one global append per list (a solo workgroup's
+  // lists start at 0)
+  const uint32_t nl = min(sm.lq_next, (uint32_t)kPushCap);
+  const uint32_t sl = min(sm.lq_sel, (uint32_t)kPushSelCap);
+  uint32_t gb_next = 0, gb_sel = 0;
+  if (!solo) {
+    // both lists' places in one 64-bit add (every workgroup of the step
+    // adds to this word: one add each, not one per list and counter)
+    if (tid == 0) {
+      unsigned long long old = 0;
+      if (nl || sl)
+        old = atomicAdd(&v.ctl->pushes, (unsigned long long)nl | ((unsigned long long)sl << 32));
+      sm.gb_next = (uint32_t)old;
+      sm.gb_sel = (uint32_t)(old >> 32);
+    }
+    __syncthreads();
+    gb_next = sm.gb_next;
+    gb_sel = sm.gb_sel;
+  }
+  const bool next_in_lds = solo && sm.lq_next <= v.keep_lds_max;
+  for (uint32_t i = tid; i < (next_in_lds ? 0u : nl); i += kBlock) {
+    const uint32_t o = gb_next + i;
+    const NextRec& r = sm.push_next[i];
+    if (o < v.next_cap) st_next(&v.nextc[o], r.key, r.node, r.jk);
+  }
+  for (uint32_t i = tid; i < sl; i += kBlock) {
+    const uint32_t o = gb_sel + i;
+    if (v.nS + o < v.sel_cap) st_sel(&v.sel[v.nS + o], sm.push_sel[i]);
+  }
+}
+
 // Expands the step's work items: each is (parent, child) for a scanned
 // parent, (parent, proposal) for a searched or hashed parent, or the single
 // pending token of a link parent.  Items go out in chunks of 64 (one per
@@ -1228,15 +1404,143 @@ __device__ __forceinline__ void cut_of_step(const KArgs& a, StepView& v, uint32_
 // step alone: its LDS counters are the list lengths and the control block is
 // not used (the counts stay in sm.lq_next, sm.lq_sel, sm.w_children and
 // sm.w_probes).
-// kLean (see tbs_kernel): the parent table and the row are in LDS, and a step
-// of many chunks is queued (queues_items).
-template <bool kLean>
 __device__ __forceinline__ void expand_range(const KArgs& a, const StepView& v, uint32_t W,
                              uint32_t gwave0, uint32_t nwaves, bool leader, bool solo,
                              bool hashed, Smem& sm) {
   const uint32_t tid = threadIdx.x, lane = tid & 63u;
-  const bool lds_par = kLean || v.n_par <= (uint32_t)kBlock;
-  const bool queued = kLean && queues_items(a, v, W, nwaves, hashed);
+  const bool lds_par = v.n_par <= (uint32_t)kBlock;
+  uint32_t my_children = 0, my_probes = 0;
+  const uint32_t K = v.K, t = v.t;
+  const uint32_t nchunks = (W + 63u) >> 6;
+  const uint32_t nwg = nwaves / (uint32_t)kWaves, slice = gwave0 / (uint32_t)kWaves;
+  for (uint32_t c = slice + nwg * (tid >> 6); c < nchunks; c += nwaves) {
+    const uint32_t w = (c << 6) + lane;
+    bool do_next = false, do_sel = false;
+    uint32_t cnode = 0, pj = 0, k = 0, tok = 0;
+    double s2 = 0.0;
+    // The chunk's parents, when the table is in LDS: those of its first and
+    // last items (pa, pb) by a 64-ary search of the prefix, two rounds of one
+    // LDS read a lane and a ballot (the prefix is non-decreasing, woff[0] is
+    // 0 and woff[n_par] is W, so each ballot is a run of low lanes); each
+    // lane then searches [pa, pb] alone -- nothing when one parent holds the
+    // whole chunk, as a hashed parent's K items mostly do.
+    uint32_t pa = 0, pb = v.n_par;
+    if (lds_par && !v.one_each) {
+      const uint32_t w0 = c << 6, wl = min(w0 + 63u, W - 1u);
+      const uint32_t st = (v.n_par + 64u) >> 6;  // 64 st > n_par
+      const uint32_t o1 = sm.woff[min(lane * st, v.n_par)];
+      const uint64_t m0 = __ballot(o1 <= w0), m1 = __ballot(o1 <= wl);
+      const uint32_t b0 = (63u - (uint32_t)__clzll((long long)m0)) * st;
+      const uint32_t b1 = (63u - (uint32_t)__clzll((long long)m1)) * st;
+      const uint64_t n0 = __ballot(lane < st && sm.woff[min(b0 + lane, v.n_par)] <= w0);
+      const uint64_t n1 = __ballot(lane < st && sm.woff[min(b1 + lane, v.n_par)] <= wl);
+      pa = b0 + (63u - (uint32_t)__clzll((long long)n0));
+      pb = b1 + (63u - (uint32_t)__clzll((long long)n1)) + 1u;
+    }
+    if (w < W) {
+      // parent of work item w: the last j with woff[j] <= w
+      uint32_t lo = pa, hi = pb;
+      if (v.one_each) {
+        lo = w;
+      } else {
+        while (hi - lo > 1) {
+          const uint32_t mid = (lo + hi) >> 1;
+          const uint32_t o = lds_par ? sm.woff[mid] : ld_relaxed(&v.woff[mid]);
+          if (o <= w) lo = mid; else hi = mid;
+        }
+      }
+      pj = lo;
+      uint32_t md, c0, aux, q;
+      if (lds_par) {
+        q = w - sm.woff[pj];
+        md = sm.p_mode[pj];
+        c0 = sm.p_c0[pj];
+        aux = sm.p_aux[pj];
+      } else {
+        q = w - ld_relaxed(&v.woff[pj]);
+        md = ld_relaxed(&v.pmode[pj]);
+        c0 = ld_relaxed(&v.pc0[pj]);
+        aux = ld_relaxed(&v.paux[pj]);
+      }
+      const bool depth_ok = (md & kModeDepthOk) != 0;
+      const bool filtered = (md & kModeFiltered) != 0;
+      md &= kModeMask;
+      int pos = -1;
+      bool have_child = false, label_sel = false;
+      // the token a link parent or a scanned child looks up in the row
+      uint32_t ftok = kNoToken;
+      if (md == M_LP_NEXT || md == M_LP_SEL) {
+        // the leader reads the next pending token of a link parent that
+        // stays one (for its emit) while the row is searched
+        uint32_t xtok = kNoToken;
+        if (leader && lds_par && md == M_LP_NEXT) {
+          const uint32_t tc = sm.p_lp[pj];
+          if (tc != kNoCursor) xtok = a.tail[tc + 1u];
+        }
+        ftok = aux;
+        cnode = lds_par ? sm.p_node[pj] : ld_relaxed(&v.pnode[pj]);
+        if (xtok != kNoToken) sm.x_tok[pj] = xtok;
+      } else if (md == M_SCAN) {
+        // the child's label: its first token, and whether it closes a key
+        cnode = c0 + q;
+        const uint32_t lw = a.labels[cnode];
+        ++my_children;
+        ftok = lw & kTokMask;
+        have_child = true;
+        label_sel = (lw & kSlotSel) && depth_ok;
+      } else if (md == M_SEARCH || md == M_HASH || md == M_DENSE) {
+        pos = (int)q;
+      }
+      if (ftok != kNoToken)
+        pos = K > kMaxLdsTopk ? grow_find((const uint32_t*)sm.grow_id, K, ftok)
+                              : row_find(sm, K, ftok, hashed);
+      if (pos >= 0) {
+        float x;
+        if (K > kMaxLdsTopk) {
+          x = __uint_as_float(ld_relaxed((const uint32_t*)sm.grow_lp + pos));
+          tok = ld_relaxed((const uint32_t*)sm.grow_id + pos);
+        } else {
+          x = sm.row_lp[pos];
+          tok = sm.row_id[pos];
+        }
+        k = (uint32_t)pos;
+        const double ps = lds_par ? sm.p_s[pj] : ld_cur(&v.cur[pj]).s;
+        // thresholds in double, `<=` drops (louds-trie.cc:87-90)
+        const bool low = ((double)x <= (double)v.tok_thr) ||
+                         (ps + (double)x <= v.sent_thr);
+        if (!low) {
+          s2 = ps + (double)x;
+          find_child(a, md, c0, aux, tok, t, depth_ok, filtered, my_probes, cnode, have_child,
+                     label_sel);
+          if (md == M_LP_NEXT) {
+            do_next = true;
+          } else if (md == M_LP_SEL) {
+            do_sel = true;
+          } else if (have_child) {
+            // a child is always next; selected when it closes a key of
+            // length t + 1 (louds-trie.cc:103-108)
+            do_next = true;
+            do_sel = label_sel;
+          }
+        }
+      }
+    }
+    append_pushes(v, do_next, do_sel, s2, cnode, pj, k, tok, lds_par, solo, sm);
+  }
+  expand_end(v, my_children, my_probes, solo, sm);
+}
+
+// expand_range of the lean instantiation (see tbs_kernel): the parent table
+// and the row are in LDS, a step of many chunks is queued (queues_items), and
+// a round may have a cut.  A function of its own: with one text for both (the
+// items in a shared lambda or loop) the general instantiation's expansion was
+// slower in every step, 52.5 -> 54.2 us a request over 128 staged requests of
+// beam 250.
+__device__ __forceinline__ void expand_lean(const KArgs& a, const StepView& v, uint32_t W,
+                             uint32_t gwave0, uint32_t nwaves, bool leader, bool solo,
+                             bool hashed, SmemLean& sm) {
+  const uint32_t tid = threadIdx.x, lane = tid & 63u;
+  const bool queued = queues_items(a, v, W, nwaves, hashed);
   uint32_t my_children = 0, my_probes = 0;
   const uint32_t K = v.K, t = v.t;
   const uint32_t nchunks = (W + 63u) >> 6;
@@ -1270,7 +1574,7 @@ __device__ __forceinline__ void expand_range(const KArgs& a, const StepView& v, 
   // otherwise loaded again, and waited for, in every round
   const uint32_t* labels = a.labels;
   const uint64_t* wfp = a.wfp;
-  if constexpr (kLean) asm volatile("" : "+s"(labels), "+s"(wfp));
+  asm volatile("" : "+s"(labels), "+s"(wfp));
   for (;;) {
     bool do_next = false, do_sel = false;
     uint32_t cnode = 0, pj = 0, k = 0, tok = 0;
@@ -1373,7 +1677,7 @@ __device__ __forceinline__ void expand_range(const KArgs& a, const StepView& v, 
       if (c >= nchunks) break;
       const uint32_t w = (c << 6) + lane;
       uint32_t pa = 0, pb = v.n_par;
-      if (lds_par && !v.one_each) chunk_parents(c, pa, pb);
+      if (!v.one_each) chunk_parents(c, pa, pb);
       c += nwaves;
       item_ok = w < W;
       if (item_ok) {
@@ -1384,25 +1688,16 @@ __device__ __forceinline__ void expand_range(const KArgs& a, const StepView& v, 
         } else {
           while (hi - lo > 1) {
             const uint32_t mid = (lo + hi) >> 1;
-            const uint32_t o = lds_par ? sm.woff[mid] : ld_relaxed(&v.woff[mid]);
-            if (o <= w) lo = mid; else hi = mid;
+            if (sm.woff[mid] <= w) lo = mid; else hi = mid;
           }
         }
         pj = lo;
-        q = w - (lds_par ? sm.woff[pj] : ld_relaxed(&v.woff[pj]));
+        q = w - sm.woff[pj];
       }
     }
     if (item_ok) {
-      uint32_t md, c0, aux;
-      if (lds_par) {
-        md = sm.p_mode[pj];
-        c0 = sm.p_c0[pj];
-        aux = sm.p_aux[pj];
-      } else {
-        md = ld_relaxed(&v.pmode[pj]);
-        c0 = ld_relaxed(&v.pc0[pj]);
-        aux = ld_relaxed(&v.paux[pj]);
-      }
+      uint32_t md = sm.p_mode[pj];
+      const uint32_t c0 = sm.p_c0[pj], aux = sm.p_aux[pj];
       const bool depth_ok = (md & kModeDepthOk) != 0;
       const bool filtered = (md & kModeFiltered) != 0;
       md &= kModeMask;
@@ -1414,12 +1709,12 @@ __device__ __forceinline__ void expand_range(const KArgs& a, const StepView& v, 
         // the leader reads the next pending token of a link parent that
         // stays one (for its emit) while the row is searched
         uint32_t xtok = kNoToken;
-        if (leader && lds_par && md == M_LP_NEXT) {
+        if (leader && md == M_LP_NEXT) {
           const uint32_t tc = sm.p_lp[pj];
           if (tc != kNoCursor) xtok = a.tail[tc + 1u];
         }
         ftok = aux;
-        cnode = lds_par ? sm.p_node[pj] : ld_relaxed(&v.pnode[pj]);
+        cnode = sm.p_node[pj];
         if (xtok != kNoToken) sm.x_tok[pj] = xtok;
       } else if (md == M_SCAN) {
         // the child's label: its first token, and whether it closes a key
@@ -1433,95 +1728,19 @@ __device__ __forceinline__ void expand_range(const KArgs& a, const StepView& v, 
         pos = (int)q;
       }
       if (ftok != kNoToken)
-        pos = !kLean && K > kMaxLdsTopk ? grow_find((const uint32_t*)sm.grow_id, K, ftok)
-                              : row_find(sm, K, ftok, hashed);
+        pos = row_find(sm, K, ftok, hashed);
       if (pos >= 0) {
-        float x;
-        if (!kLean && K > kMaxLdsTopk) {
-          x = __uint_as_float(ld_relaxed((const uint32_t*)sm.grow_lp + pos));
-          tok = ld_relaxed((const uint32_t*)sm.grow_id + pos);
-        } else {
-          x = sm.row_lp[pos];
-          tok = sm.row_id[pos];
-        }
+        const float x = sm.row_lp[pos];
+        tok = sm.row_id[pos];
         k = (uint32_t)pos;
-        const double ps = lds_par ? sm.p_s[pj] : ld_cur(&v.cur[pj]).s;
+        const double ps = sm.p_s[pj];
         // thresholds in double, `<=` drops (louds-trie.cc:87-90)
         const bool low = ((double)x <= (double)v.tok_thr) ||
                          (ps + (double)x <= v.sent_thr);
         if (!low) {
           s2 = ps + (double)x;
-          if (md == M_SEARCH) {
-            // lower_bound of tok among the parent's children
-            uint32_t lo2 = c0, hi2 = c0 + aux;
-            const uint32_t end2 = hi2;
-            while (lo2 < hi2) {
-              const uint32_t mid = lo2 + ((hi2 - lo2) >> 1);
-              ++my_probes;
-              if (a.recs[mid].first_tok < tok) lo2 = mid + 1; else hi2 = mid;
-            }
-            if (lo2 < end2) {
-              const ft_node_rec cr = a.recs[lo2];
-              if (cr.first_tok == tok) {
-                cnode = lo2;
-                have_child = true;
-                // terminal with |KB| == |Q| -> selected (louds-trie.cc:103-108)
-                label_sel = (cr.meta & FT_META_TERMINAL) &&
-                            (cr.meta & FT_META_DEPTH_MASK) == t + 1;
-              }
-            }
-          } else if (md == M_HASH) {
-            // the token's first cuckoo bucket, and its second only when the
-            // first is full without a match
-            const uint32_t lg = aux;
-            uint32_t b = c0 + cuckoo_h1(tok, lg);
-            // a filtered table: no fingerprint match in the first bucket
-            // (nor in the second, when the first is full) means no child
-            bool maybe = true;
-            if (filtered && !matched) {
-              const uint64_t f8 = (uint64_t)wide_fp(tok) * 0x0101010101010101ull;
-              const uint64_t w1 = a.wfp[b];
-              maybe = has_zero_byte(w1 ^ f8);
-              if (!maybe && !has_zero_byte(w1))
-                maybe = has_zero_byte(a.wfp[c0 + cuckoo_h2(tok, lg)] ^ f8);
-            }
-            uint32_t hw = 0, hc = 0;
-            for (int round = 0; round < (maybe ? 2 : 0); ++round) {
-              // the whole bucket (tokens and children) in one read
-              const uint4* bw = (const uint4*)&a.wtab[b];
-              const uint4 ta = bw[0], tb = bw[1], ca = bw[2], cb = bw[3];
-              ++my_probes;
-              const uint32_t tw[8] = {ta.x, ta.y, ta.z, ta.w, tb.x, tb.y, tb.z, tb.w};
-              const uint32_t cw[8] = {ca.x, ca.y, ca.z, ca.w, cb.x, cb.y, cb.z, cb.w};
-              bool full = true;
-#pragma unroll
-              for (int sl = 0; sl < 8; ++sl) {
-                if ((tw[sl] & kTokMask) == tok) {
-                  hw = tw[sl];
-                  hc = cw[sl];
-                }
-                full = full && tw[sl] != kSlotEmptyTok;
-              }
-              if (hc != 0u || !full) break;
-              b = c0 + cuckoo_h2(tok, lg);
-            }
-            if (hc != 0u) {
-              cnode = hc;
-              have_child = true;
-              label_sel = (hw & kSlotSel) && depth_ok;
-            }
-          } else if (md == M_DENSE) {
-            // the root's child of this token: one read of (node, flags)
-            if (tok < a.root_n) {
-              const uint2 rd = *(const uint2*)&a.root_dir[tok];
-              ++my_probes;
-              if (rd.x != 0u) {
-                cnode = rd.x;
-                have_child = true;
-                label_sel = (rd.y & kRdSel) && depth_ok;
-              }
-            }
-          }
+          find_child(a, md, c0, aux, tok, t, depth_ok, filtered && !matched, my_probes, cnode,
+                     have_child, label_sel);
           if (md == M_LP_NEXT) {
             do_next = true;
           } else if (md == M_LP_SEL) {
@@ -1532,7 +1751,7 @@ __device__ __forceinline__ void expand_range(const KArgs& a, const StepView& v, 
             do_next = true;
             do_sel = label_sel;
           }
-          if (kLean && v.cut_mode != kCutNone) {
+          if (v.cut_mode != kCutNone) {
             const bool above = s2 * v.lnf_next >= v.cut;
             do_next = do_next && above == (v.cut_mode == kCutAbove);
             do_sel = do_sel && v.cut_mode == kCutAbove;
@@ -1540,81 +1759,9 @@ __device__ __forceinline__ void expand_range(const KArgs& a, const StepView& v, 
         }
       }
     }
-    // appends (every lane of the wave reaches these): into the LDS
-    // buffers while they have room, the rest straight to the global lists
-    const uint32_t jk = (pj << 16) | k;
-    if (__ballot(do_next)) {
-      const uint32_t li = wave_append(do_next, &sm.lq_next);
-      const bool spill = do_next && li >= (uint32_t)kPushCap;
-      const uint32_t gi = solo ? li : wave_append_half(spill, &v.ctl->pushes, false);
-      if (do_next) {
-        const uint64_t key = norm_key(s2 * v.lnf_next);
-        if (!spill) {
-          sm.push_next[li].key = key;
-          sm.push_next[li].node = cnode;
-          sm.push_next[li].jk = jk;
-        } else if (gi < v.next_cap) {
-          st_next(&v.nextc[gi], key, cnode, jk);
-        }
-      }
-    }
-    if (__ballot(do_sel)) {
-      const uint32_t li = wave_append(do_sel, &sm.lq_sel);
-      const bool spill = do_sel && li >= (uint32_t)kPushSelCap;
-      const uint32_t gi = solo ? li : wave_append_half(spill, &v.ctl->pushes, true);
-      if (do_sel) {
-        SelRec sr;
-        sr.s = s2;
-        sr.node = cnode;
-        sr.depth = t + 1;
-        sr.phist = lds_par ? sm.p_hist[pj] : ld_cur(&v.cur[pj]).hist;
-        sr.tok = tok;
-        sr.jk = jk;
-        sr.isnew = 1;
-        if (!spill) sm.push_sel[li] = sr;
-        else if (v.nS + gi < v.sel_cap) st_sel(&v.sel[v.nS + gi], sr);
-      }
-    }
+    append_pushes(v, do_next, do_sel, s2, cnode, pj, k, tok, true, solo, sm);
   }
-  // the workgroup's counters: one LDS add a wave (lane by lane, the adds to
-  // one word would run one after another, 1024 of them)
-  {
-    const uint32_t wc = wave_sum(my_children), wp = wave_sum(my_probes);
-    if ((tid & 63u) == 0u) {
-      if (wc) atomicAdd(&sm.w_children, wc);
-      if (wp) atomicAdd(&sm.w_probes, wp);
-    }
-  }
-  __syncthreads();
-  // the buffered pushes: one global append per list (a solo workgroup's
-  // lists start at 0)
-  const uint32_t nl = min(sm.lq_next, (uint32_t)kPushCap);
-  const uint32_t sl = min(sm.lq_sel, (uint32_t)kPushSelCap);
-  uint32_t gb_next = 0, gb_sel = 0;
-  if (!solo) {
-    // both lists' places in one 64-bit add (every workgroup of the step
-    // adds to this word: one add each, not one per list and counter)
-    if (tid == 0) {
-      unsigned long long old = 0;
-      if (nl || sl)
-        old = atomicAdd(&v.ctl->pushes, (unsigned long long)nl | ((unsigned long long)sl << 32));
-      sm.gb_next = (uint32_t)old;
-      sm.gb_sel = (uint32_t)(old >> 32);
-    }
-    __syncthreads();
-    gb_next = sm.gb_next;
-    gb_sel = sm.gb_sel;
-  }
-  const bool next_in_lds = solo && sm.lq_next <= v.keep_lds_max;
-  for (uint32_t i = tid; i < (next_in_lds ? 0u : nl); i += kBlock) {
-    const uint32_t o = gb_next + i;
-    const NextRec& r = sm.push_next[i];
-    if (o < v.next_cap) st_next(&v.nextc[o], r.key, r.node, r.jk);
-  }
-  for (uint32_t i = tid; i < sl; i += kBlock) {
-    const uint32_t o = gb_sel + i;
-    if (v.nS + o < v.sel_cap) st_sel(&v.sel[v.nS + o], sm.push_sel[i]);
-  }
+  expand_end(v, my_children, my_probes, solo, sm);
 }
 
 // Loads the proposal row of step t (staged in ascending token order) into
@@ -1636,14 +1783,14 @@ __device__ __forceinline__ void load_row(const uint32_t* rid, const float* rlp, 
 // insert ends in a free slot.
 // kBits: the row's token bits (kRowBits) too, which the queued steps look at.
 template <bool kBits>
-__device__ __forceinline__ void row_hash_clear(Smem& sm) {
+__device__ __forceinline__ void row_hash_clear(SmemOf<kBits>& sm) {
   for (uint32_t i = threadIdx.x; i < (uint32_t)kRowHash; i += kBlock)
     sm.rh_tok[i] = kRowHashEmpty;
   if constexpr (kBits)
     for (uint32_t i = threadIdx.x; i < kRowBits / 32u; i += kBlock) sm.rh_bits[i] = 0u;
 }
 template <bool kBits>
-__device__ __forceinline__ void row_hash_insert(uint32_t tok, uint32_t p, Smem& sm) {
+__device__ __forceinline__ void row_hash_insert(uint32_t tok, uint32_t p, SmemOf<kBits>& sm) {
   if (tok >= kTokMask) return;
   if constexpr (kBits) {
     const uint32_t bit = row_bit(tok);
@@ -1662,7 +1809,7 @@ __device__ __forceinline__ void row_hash_insert(uint32_t tok, uint32_t p, Smem& 
 // Hashes the LDS row (the workgroup has synchronised since the row was
 // written).  Ends synchronised.
 template <bool kBits>
-__device__ __forceinline__ void hash_row(uint32_t K, Smem& sm) {
+__device__ __forceinline__ void hash_row(uint32_t K, SmemOf<kBits>& sm) {
   row_hash_clear<kBits>(sm);
   __syncthreads();
   for (uint32_t p = threadIdx.x; p < K; p += kBlock) row_hash_insert<kBits>(sm.row_id[p], p, sm);
@@ -1943,7 +2090,7 @@ __device__ __forceinline__ bool ensure_rows(const KArgs& a, uint32_t req, const 
 // slice of the work items, until the leader posts the exit generation.
 template <bool kStreamed, bool kLean>
 __device__ __forceinline__ void helper_loop(const KArgs& a, const DevReq& d, uint8_t* ws,
-                            uint32_t g, Smem& sm) {
+                            uint32_t g, SmemOf<kLean>& sm) {
   const uint32_t tid = threadIdx.x;
   Ctl* ctl = (Ctl*)(ws + a.lay.ctl);
   const unsigned long long tag = (unsigned long long)a.epoch << 32;
@@ -2032,8 +2179,10 @@ __device__ __forceinline__ void helper_loop(const KArgs& a, const DevReq& d, uin
         sm.hstep[1] = pW;
         sm.hstep[2] = pn;
         sm.hstep[3] = pS;
-        sm.hcut = ld_relaxed(&ctl->cut);
-        sm.hcut_mode = ld_relaxed(&ctl->cut_mode);
+        if constexpr (kLean) {
+          sm.hcut = ld_relaxed(&ctl->cut);
+          sm.hcut_mode = ld_relaxed(&ctl->cut_mode);
+        }
         sm.hstep[4] = ld_relaxed(&ctl->cur_which);
         sm.hstep[5] = ld_relaxed(&ctl->sel_which);
         // A posted step always satisfies the bounds below; a claimed slice
@@ -2048,8 +2197,13 @@ __device__ __forceinline__ void helper_loop(const KArgs& a, const DevReq& d, uin
     const unsigned long long v = sm.bcast;
     const uint32_t t = sm.hstep[0], W = sm.hstep[1], n_par = sm.hstep[2],
                    nS = sm.hstep[3], cur_which = sm.hstep[4], sel_which = sm.hstep[5];
-    const uint32_t mine = sm.hstep[6], cut_mode = sm.hcut_mode;
-    const double cut = __longlong_as_double((long long)sm.hcut);
+    const uint32_t mine = sm.hstep[6];
+    double cut = 0.0;
+    uint32_t cut_mode = kCutNone;
+    if constexpr (kLean) {
+      cut = __longlong_as_double((long long)sm.hcut);
+      cut_mode = sm.hcut_mode;
+    }
     __syncthreads();
     if ((v >> 32) != a.epoch || (uint32_t)v == kGoExit || v == seen) return;
     seen = v;
@@ -2143,8 +2297,12 @@ __device__ __forceinline__ void helper_loop(const KArgs& a, const DevReq& d, uin
       sm.lq_sel = 0;
     }
     __syncthreads();
-    expand_range<kLean>(a, sv, W, g * (uint32_t)kWaves, a.wgs * (uint32_t)kWaves, false, false,
-                        hashed, sm);
+    if constexpr (kLean)
+      expand_lean(a, sv, W, g * (uint32_t)kWaves, a.wgs * (uint32_t)kWaves, false, false,
+                  hashed, sm);
+    else
+      expand_range(a, sv, W, g * (uint32_t)kWaves, a.wgs * (uint32_t)kWaves, false, false,
+                   hashed, sm);
     // the row lookups are done: empty the hash for the next step
     if (hashed) row_hash_clear<kLean>(sm);
     if (tid == 0) st_dev(dw + 1, pack2(sm.w_children, sm.w_probes));
@@ -2450,7 +2608,7 @@ __device__ __forceinline__ void tiny_steps(
     hist_used += n_next;
     nS += n_new;
     cands += (uint64_t)n_next + n_new;
-    if (lane == 0) lds_add(&sm.cnt_parents, n_cur);
+    if (lane == 0) sm.cnt_parents += n_cur;
     n_cur = n_next;
     ticks += c1 - c0;
     c0 = c1;
@@ -2505,13 +2663,15 @@ __device__ __forceinline__ void tiny_steps(
 // kLean: every beam and row of the launch is at most kBlock long (launch_tbs
 // is told), so that the parent table and the row of a step are always in LDS,
 // one thread an entry.  The instantiation leaves out the code for longer ones
-// and queues the items of large steps: 100 KB of code against 117 KB with
+// and queues the items of large steps: 103 KB of code against 117 KB with
 // neither, which pays at every step since the leader's loop does not fit the
 // 64 KB instruction cache (the queue beside the general code made calls of
-// batch 1 3-5% slower).
+// batch 1 3-5% slower).  The general one shares the functions but not the text
+// of a step's expansion (expand_range, expand_lean): small calls are as fast
+// with it as they were without the lean one.
 template <bool kLouds, bool kStreamed, bool kLean>
 __global__ void __launch_bounds__(kBlock) tbs_kernel(KArgs a) {
-  __shared__ Smem sm;
+  __shared__ SmemOf<kLean> sm;
   // request-major interleave: request r owns blocks r, r + batch, ...  The
   // dispatcher deals blocks to the 8 XCDs round-robin, so at batch 8 each
   // request's workgroups share one XCD and its L2.
@@ -2590,8 +2750,13 @@ __global__ void __launch_bounds__(kBlock) tbs_kernel(KArgs a) {
                  hist_cap = a.lay.hist_cap;
   const unsigned long long tag = (unsigned long long)a.epoch << 32;
   uint32_t gen = 0;
+  unsigned long long t_post = 0;  // (thread 0) wall clock of the last post
 
-  if (tid == 0) sm.t_all0 = wall_clock64();
+  // (the lean instantiation's clocks and its candidates are in LDS)
+  unsigned long long t_exp = 0, t_sel = 0, t_all0 = wall_clock64();
+  if constexpr (kLean) {
+    if (tid == 0) sm.t_all0 = t_all0;
+  }
   // per-step profile rows after the output tokens: kStepStats u64 per step
   uint64_t* step_stats = (uint64_t*)(ob + step_stats_offset(d.F, d.out_T));
   for (uint32_t i = tid; i < d.out_T * kStepStats; i += kBlock) step_stats[i] = 0;
@@ -2600,9 +2765,10 @@ __global__ void __launch_bounds__(kBlock) tbs_kernel(KArgs a) {
     sm.status = 0;
     sm.multi_item = 0;
     sm.cnt_parents = sm.cnt_children = sm.cnt_probes = 0;
-    sm.t_exp = sm.t_sel = sm.n_cands = 0;
+    if constexpr (kLean) sm.t_exp = sm.t_sel = sm.n_cands = 0;
   }
   uint32_t n_cur = 1, nS = 0, hist_used = 0;
+  uint64_t n_cands = 0;
   // the parent table of the step was written by the previous step's emit,
   // and its row loaded into registers there (pf_*); for step 0 both are
   // read here, the root's entry by one thread of wave 1 while every thread
@@ -2616,7 +2782,7 @@ __global__ void __launch_bounds__(kBlock) tbs_kernel(KArgs a) {
   }
   uint32_t root_err = 0;
   if (tid == 64u) {
-    ParEntry e = parent_entry<kLouds>(a, 0u, 0u, K, &root_err);
+    ParEntry e = parent_entry<kLouds, kLean>(a, 0u, 0u, K, &root_err);
     if (a.root_dir) {
       // a root searched or hashed (or scanned, when forced) looks its
       // children up in the root directory instead; a one-token child
@@ -2682,9 +2848,14 @@ __global__ void __launch_bounds__(kBlock) tbs_kernel(KArgs a) {
           n_cur = sm.tiny_ncur;
           nS = sm.tiny_nS;
           hist_used = sm.tiny_hist;
-          if (tid == 0) {
-            lds_add(&sm.n_cands, sm.tiny_cands);
-            lds_add(&sm.t_exp, sm.tiny_ticks);
+          if constexpr (kLean) {
+            if (tid == 0) {
+              lds_add(&sm.n_cands, sm.tiny_cands);
+              lds_add(&sm.t_exp, sm.tiny_ticks);
+            }
+          } else {
+            n_cands += sm.tiny_cands;
+            t_exp += sm.tiny_ticks;
           }
           if (sm.tiny_done || sm.status) {
             finished = true;
@@ -2743,7 +2914,7 @@ __global__ void __launch_bounds__(kBlock) tbs_kernel(KArgs a) {
       }
       const CurRec p = cur[j];
       uint32_t err = 0;
-      const ParEntry e = parent_entry<kLouds>(a, p.node, t, K, &err);
+      const ParEntry e = parent_entry<kLouds, kLean>(a, p.node, t, K, &err);
       if (err) atomicOr(&sm.status, (uint32_t)kStatusCorrupt);
       st_dev(&par_c0[j], e.c0);
       st_dev(&par_aux[j], e.aux);
@@ -2805,7 +2976,8 @@ __global__ void __launch_bounds__(kBlock) tbs_kernel(KArgs a) {
       }
     }
     if (tid == 0) {
-      lds_add(&sm.cnt_parents, n_cur);
+      if constexpr (kLean) lds_add(&sm.cnt_parents, n_cur);
+      else sm.cnt_parents += n_cur;
       // this workgroup's expansion counters (expand_range of the leader
       // relies on them being zero)
       sm.w_children = 0;
@@ -2842,24 +3014,15 @@ __global__ void __launch_bounds__(kBlock) tbs_kernel(KArgs a) {
     const bool shared = a.wgs > 1 && W >= a.share_min;
     sv.cut = 0.0;
     sv.cut_mode = kCutNone;
-    const bool hashed = (kLean || K <= kRowHashMaxK) && W >= kRowHashMinWork;
-    if (kLean && shared && queues_items(a, sv, W, a.wgs * (uint32_t)kWaves, hashed))
-      cut_of_step(a, sv, beams[t], (const uint64_t*)(in + d.kb_off) + 2ull * t, sm);
-    // the leader's slice 0, then (shared) the slices it takes over: one call
-    // of the inlined expansion for both, which keeps its code and registers
-    // to one copy
     uint32_t sh_next = 0, sh_sel = 0;  // (shared) the pushes of the step
-    uint32_t lead_ch = 0, lead_pr = 0;  // the counters of the leader's slices
-    uint32_t n_stolen = 0;
-    bool stole = false;  // (thread i) slice i + 1 was taken over here
-    const uint32_t nh = a.wgs - 1;  // helper slots 1 .. nh (nh < kBlock)
-    // one round, or two when a cut let too few pushes through
-    for (;;) {
+    // The step's expansion, of the two instantiations apart (see expand_lean):
+    // one text for both cost the general one's small calls 1-2%.
+    if constexpr (!kLean) {
       if (shared) {
         // publish the step (the helpers read the row from the staged request),
         // then wake the helpers
         if (tid == 0) {
-          if (sv.cut_mode != kCutBelow) st_dev(&ctl->pushes, 0ull);
+          st_dev(&ctl->pushes, 0ull);
           st_dev(&ctl->t, t);
           st_dev(&ctl->W, W);
           st_dev(&ctl->n_par, n_cur);
@@ -2867,20 +3030,19 @@ __global__ void __launch_bounds__(kBlock) tbs_kernel(KArgs a) {
           st_dev(&ctl->sel_which, sel_which);
           st_dev(&ctl->cur_which, cur_which);
           st_dev(&ctl->hist_n, hist_used);
-          st_dev(&ctl->cut, (unsigned long long)__double_as_longlong(sv.cut));
-          st_dev(&ctl->cut_mode, sv.cut_mode);
         }
         wait_stores();  // the step's data is complete before `go` moves
         __syncthreads();
         ++gen;
         if (tid == 0) {
           st_dev(&ctl->go, tag | gen);
-          sm.t_post = wall_clock64();
+          t_post = wall_clock64();
         }
       }
       // (the parent table ended synchronised: the row and the emptied hash are
       // visible)
-      if (hashed && sv.cut_mode != kCutBelow) hash_row<kLean>(K, sm);
+      const bool hashed = K <= kRowHashMaxK && W >= kRowHashMinWork;
+      if (hashed) hash_row<false>(K, sm);
       // (streamed) helper 1 copying the request's later rows claims no slice
       // meanwhile: its slice is taken over at once rather than after the
       // grace period (thread 0 stands for slot 1 below)
@@ -2889,56 +3051,259 @@ __global__ void __launch_bounds__(kBlock) tbs_kernel(KArgs a) {
         if (shared && tid == 0 && !ss.done && !ss.own && ss.split < T)
           copying1 = ld_relaxed(&ctl->copy) == (tag | kCopyClaimed);
       }
-      const unsigned long long mygo = tag | gen;
-      for (uint32_t taken = 0, slice = 0;;) {
-        expand_range<kLean>(a, sv, W, slice * (uint32_t)kWaves,
-                            (shared ? a.wgs : 1u) * (uint32_t)kWaves, true, !shared, hashed, sm);
-        lead_ch += sm.w_children;
-        lead_pr += sm.w_probes;
-        if (!shared) break;
-        if (slice == 0) {
-          // The helpers' slices: each is claimed by its helper (its claim word
-          // set to this step) or, once kGraceTicks have passed since the post,
-          // taken over here -- so the step never waits for a workgroup that is
-          // not running.  Then every claimed slice is waited for: a helper that
-          // claimed one is running and finishes it.
-          if (tid == 0) sm.t_wait = wall_clock64();
-          unsigned long long* claims = (unsigned long long*)(ws + a.lay.claims);
-          bool pending_any = true;
-          for (;;) {
-            const int pending = __syncthreads_count(tid < nh && !copying1 &&
-                                                    ld_relaxed(&claims[tid + 1]) != mygo);
-            if (pending == 0) {
-              pending_any = false;
-              break;
-            }
-            if (tid == 0) sm.lead_flag = (wall_clock64() - sm.t_post > kGraceTicks) ? 1u : 0u;
-            __syncthreads();
-            const bool expired = sm.lead_flag != 0;
-            __syncthreads();
-            if (expired) break;
-            __builtin_amdgcn_s_sleep(2);
+      expand_range(a, sv, W, 0, (shared ? a.wgs : 1u) * (uint32_t)kWaves, true, !shared,
+                   hashed, sm);
+      // the counters of the leader's slices
+      uint32_t lead_ch = sm.w_children, lead_pr = sm.w_probes;
+      if (shared) {
+        // The helpers' slices: each is claimed by its helper (its claim word
+        // set to this step) or, once kGraceTicks have passed since the post,
+        // taken over here -- so the step never waits for a workgroup that is
+        // not running.  Then every claimed slice is waited for: a helper that
+        // claimed one is running and finishes it.
+        const unsigned long long tw0 = wall_clock64();
+        const unsigned long long mygo = tag | gen;
+        unsigned long long* claims = (unsigned long long*)(ws + a.lay.claims);
+        const uint32_t nh = a.wgs - 1;  // helper slots 1 .. nh (nh < kBlock)
+        bool pending_any = true;
+        for (;;) {
+          const int pending = __syncthreads_count(tid < nh && !copying1 &&
+                                                  ld_relaxed(&claims[tid + 1]) != mygo);
+          if (pending == 0) {
+            pending_any = false;
+            break;
           }
-          // (thread 0 alone knows whether helper 1 is copying: the takeover
-          // runs when any slot is still pending or helper 1 copies)
-          if (__syncthreads_or(pending_any || copying1)) {
-            if (tid == 0) sm.n_stolen = 0;
-            __syncthreads();
-            // raise every unclaimed word (helper 1's alone when only it is
-            // copying): a slice whose word this raises is taken over here; one
-            // a helper raised first stays the helper's
-            if (tid < nh && (pending_any || tid == 0) &&
-                atomicMax(&claims[tid + 1], mygo) < mygo) {
-              stole = true;
-              const uint32_t k = atomicAdd(&sm.n_stolen, 1u);
-              sm.stolen[k] = (uint16_t)(tid + 1);
-            }
-            __syncthreads();
-            n_stolen = sm.n_stolen;
+          if (tid == 0) sm.lead_flag = (wall_clock64() - t_post > kGraceTicks) ? 1u : 0u;
+          __syncthreads();
+          const bool expired = sm.lead_flag != 0;
+          __syncthreads();
+          if (expired) break;
+          __builtin_amdgcn_s_sleep(2);
+        }
+        uint32_t n_stolen = 0;
+        bool stole = false;  // (thread i) slice i + 1 was taken over here
+        // (thread 0 alone knows whether helper 1 is copying: the takeover
+        // runs when any slot is still pending or helper 1 copies)
+        if (__syncthreads_or(pending_any || copying1)) {
+          if (tid == 0) sm.n_stolen = 0;
+          __syncthreads();
+          // raise every unclaimed word (helper 1's alone when only it is
+          // copying): a slice whose word this raises is taken over here; one
+          // a helper raised first stays the helper's
+          if (tid < nh && (pending_any || tid == 0) &&
+              atomicMax(&claims[tid + 1], mygo) < mygo) {
+            stole = true;
+            const uint32_t k = atomicAdd(&sm.n_stolen, 1u);
+            sm.stolen[k] = (uint16_t)(tid + 1);
+          }
+          __syncthreads();
+          n_stolen = sm.n_stolen;
+        }
+        for (uint32_t i = 0; i < n_stolen; ++i) {
+          const uint32_t slice = sm.stolen[i];
+          __syncthreads();
+          if (tid == 0) {
+            sm.w_children = 0;
+            sm.w_probes = 0;
+            sm.lq_next = 0;
+            sm.lq_sel = 0;
+          }
+          __syncthreads();
+          expand_range(a, sv, W, slice * (uint32_t)kWaves, a.wgs * (uint32_t)kWaves, true, false,
+                       hashed, sm);
+          lead_ch += sm.w_children;
+          lead_pr += sm.w_probes;
+        }
+        // Every slice a helper claimed: thread i waits for helper i + 1's done
+        // word to carry this step's tag (written after its pushes and its
+        // counters are complete), unless thread i took that slice over.
+        const unsigned long long tw1 = wall_clock64();
+        unsigned long long* dones = (unsigned long long*)(ws + a.lay.dones);
+        const bool waits = tid < nh && !stole;
+        bool all_done = false;
+        for (uint32_t it = 0; it < kSpinLimit; ++it) {
+          if (__syncthreads_count(waits && ld_relaxed(&dones[2 * (tid + 1)]) != mygo) == 0) {
+            all_done = true;
+            break;
+          }
+          __builtin_amdgcn_s_sleep(1);
+        }
+        if (tid == 0) {
+          if (!all_done) sm.status |= kStatusCorrupt;
+          if (t < d.out_T) {
+            uint64_t* row = step_stats + (uint64_t)t * kStepStats;
+            row[8] = tw1 - tw0;
+            row[9] = wall_clock64() - tw1;
           }
         }
-        if (taken == n_stolen) break;
-        slice = sm.stolen[taken++];
+        // the helpers' counters and the step's push counts, read together
+        const unsigned long long cw = waits ? ld_relaxed(&dones[2 * (tid + 1) + 1]) : 0ull;
+        const unsigned long long pw = ld_relaxed(&ctl->pushes);
+        sh_next = (uint32_t)pw;
+        sh_sel = (uint32_t)(pw >> 32);
+        const uint32_t wc = wave_sum((uint32_t)cw), wp = wave_sum((uint32_t)(cw >> 32));
+        if (tid == 0) {
+          sm.w_children = lead_ch;
+          sm.w_probes = lead_pr;
+        }
+        __syncthreads();
+        if ((tid & 63u) == 0u) {
+          if (wc) atomicAdd(&sm.w_children, wc);
+          if (wp) atomicAdd(&sm.w_probes, wp);
+        }
+      }
+    } else {
+      const bool hashed = W >= kRowHashMinWork;
+      if (shared && queues_items(a, sv, W, a.wgs * (uint32_t)kWaves, hashed))
+        cut_of_step(a, sv, beams[t], (const uint64_t*)(in + d.kb_off) + 2ull * t, sm);
+      // the leader's slice 0, then (shared) the slices it takes over: one call
+      // of the inlined expansion for both, which keeps its code and registers
+      // to one copy
+      uint32_t lead_ch = 0, lead_pr = 0;  // the counters of the leader's slices
+      uint32_t n_stolen = 0;
+      bool stole = false;  // (thread i) slice i + 1 was taken over here
+      const uint32_t nh = a.wgs - 1;  // helper slots 1 .. nh (nh < kBlock)
+      // one round, or two when a cut let too few pushes through
+      for (;;) {
+        if (shared) {
+          // publish the step (the helpers read the row from the staged request),
+          // then wake the helpers
+          if (tid == 0) {
+            if (sv.cut_mode != kCutBelow) st_dev(&ctl->pushes, 0ull);
+            st_dev(&ctl->t, t);
+            st_dev(&ctl->W, W);
+            st_dev(&ctl->n_par, n_cur);
+            st_dev(&ctl->nS, nS);
+            st_dev(&ctl->sel_which, sel_which);
+            st_dev(&ctl->cur_which, cur_which);
+            st_dev(&ctl->hist_n, hist_used);
+            st_dev(&ctl->cut, (unsigned long long)__double_as_longlong(sv.cut));
+            st_dev(&ctl->cut_mode, sv.cut_mode);
+          }
+          wait_stores();  // the step's data is complete before `go` moves
+          __syncthreads();
+          ++gen;
+          if (tid == 0) {
+            st_dev(&ctl->go, tag | gen);
+            sm.t_post = wall_clock64();
+          }
+        }
+        // (the parent table ended synchronised: the row and the emptied hash are
+        // visible)
+        if (hashed && sv.cut_mode != kCutBelow) hash_row<true>(K, sm);
+        // (streamed) helper 1 copying the request's later rows claims no slice
+        // meanwhile: its slice is taken over at once rather than after the
+        // grace period (thread 0 stands for slot 1 below)
+        bool copying1 = false;
+        if constexpr (kStreamed) {
+          if (shared && tid == 0 && !ss.done && !ss.own && ss.split < T)
+            copying1 = ld_relaxed(&ctl->copy) == (tag | kCopyClaimed);
+        }
+        const unsigned long long mygo = tag | gen;
+        for (uint32_t taken = 0, slice = 0;;) {
+          expand_lean(a, sv, W, slice * (uint32_t)kWaves,
+                      (shared ? a.wgs : 1u) * (uint32_t)kWaves, true, !shared, hashed, sm);
+          lead_ch += sm.w_children;
+          lead_pr += sm.w_probes;
+          if (!shared) break;
+          if (slice == 0) {
+            // The helpers' slices: each is claimed by its helper (its claim word
+            // set to this step) or, once kGraceTicks have passed since the post,
+            // taken over here -- so the step never waits for a workgroup that is
+            // not running.  Then every claimed slice is waited for: a helper that
+            // claimed one is running and finishes it.
+            if (tid == 0) sm.t_wait = wall_clock64();
+            unsigned long long* claims = (unsigned long long*)(ws + a.lay.claims);
+            bool pending_any = true;
+            for (;;) {
+              const int pending = __syncthreads_count(tid < nh && !copying1 &&
+                                                      ld_relaxed(&claims[tid + 1]) != mygo);
+              if (pending == 0) {
+                pending_any = false;
+                break;
+              }
+              if (tid == 0) sm.lead_flag = (wall_clock64() - sm.t_post > kGraceTicks) ? 1u : 0u;
+              __syncthreads();
+              const bool expired = sm.lead_flag != 0;
+              __syncthreads();
+              if (expired) break;
+              __builtin_amdgcn_s_sleep(2);
+            }
+            // (thread 0 alone knows whether helper 1 is copying: the takeover
+            // runs when any slot is still pending or helper 1 copies)
+            if (__syncthreads_or(pending_any || copying1)) {
+              if (tid == 0) sm.n_stolen = 0;
+              __syncthreads();
+              // raise every unclaimed word (helper 1's alone when only it is
+              // copying): a slice whose word this raises is taken over here; one
+              // a helper raised first stays the helper's
+              if (tid < nh && (pending_any || tid == 0) &&
+                  atomicMax(&claims[tid + 1], mygo) < mygo) {
+                stole = true;
+                const uint32_t k = atomicAdd(&sm.n_stolen, 1u);
+                sm.stolen[k] = (uint16_t)(tid + 1);
+              }
+              __syncthreads();
+              n_stolen = sm.n_stolen;
+            }
+          }
+          if (taken == n_stolen) break;
+          slice = sm.stolen[taken++];
+          __syncthreads();
+          if (tid == 0) {
+            sm.w_children = 0;
+            sm.w_probes = 0;
+            sm.lq_next = 0;
+            sm.lq_sel = 0;
+          }
+          __syncthreads();
+        }
+        if (!shared) break;
+        // Every slice a helper claimed: thread i waits for helper i + 1's done
+        // word to carry this step's tag (written after its pushes and its
+        // counters are complete), unless thread i took that slice over.
+        const unsigned long long tw1 = wall_clock64();
+        unsigned long long* dones = (unsigned long long*)(ws + a.lay.dones);
+        const bool waits = tid < nh && !stole;
+        bool all_done = false;
+        for (uint32_t it = 0; it < kSpinLimit; ++it) {
+          if (__syncthreads_count(waits && ld_relaxed(&dones[2 * (tid + 1)]) != mygo) == 0) {
+            all_done = true;
+            break;
+          }
+          __builtin_amdgcn_s_sleep(1);
+        }
+        if (tid == 0) {
+          if (!all_done) sm.status |= kStatusCorrupt;
+          if (t < d.out_T) {
+            uint64_t* row = step_stats + (uint64_t)t * kStepStats;
+            row[8] = tw1 - sm.t_wait;
+            row[9] = wall_clock64() - tw1;
+          }
+        }
+        // the helpers' counters and the step's push counts, read together
+        const unsigned long long cw = waits ? ld_relaxed(&dones[2 * (tid + 1) + 1]) : 0ull;
+        const unsigned long long pw = ld_relaxed(&ctl->pushes);
+        sh_next = (uint32_t)pw;
+        sh_sel = (uint32_t)(pw >> 32);
+        const uint32_t wc = wave_sum((uint32_t)cw), wp = wave_sum((uint32_t)(cw >> 32));
+        if (tid == 0) {
+          sm.w_children = lead_ch;
+          sm.w_probes = lead_pr;
+        }
+        __syncthreads();
+        if ((tid & 63u) == 0u) {
+          if (wc) atomicAdd(&sm.w_children, wc);
+          if (wp) atomicAdd(&sm.w_probes, wp);
+        }
+        if (sv.cut_mode != kCutAbove || sh_next >= beams[t] || !all_done) break;
+        // too few pushes reach the cut: the others, in a second round
+        sv.cut_mode = kCutBelow;
+        __syncthreads();
+        lead_ch = sm.w_children;
+        lead_pr = sm.w_probes;
+        n_stolen = 0;
+        stole = false;
         __syncthreads();
         if (tid == 0) {
           sm.w_children = 0;
@@ -2946,60 +3311,6 @@ __global__ void __launch_bounds__(kBlock) tbs_kernel(KArgs a) {
           sm.lq_next = 0;
           sm.lq_sel = 0;
         }
-        __syncthreads();
-      }
-      if (!shared) break;
-      // Every slice a helper claimed: thread i waits for helper i + 1's done
-      // word to carry this step's tag (written after its pushes and its
-      // counters are complete), unless thread i took that slice over.
-      const unsigned long long tw1 = wall_clock64();
-      unsigned long long* dones = (unsigned long long*)(ws + a.lay.dones);
-      const bool waits = tid < nh && !stole;
-      bool all_done = false;
-      for (uint32_t it = 0; it < kSpinLimit; ++it) {
-        if (__syncthreads_count(waits && ld_relaxed(&dones[2 * (tid + 1)]) != mygo) == 0) {
-          all_done = true;
-          break;
-        }
-        __builtin_amdgcn_s_sleep(1);
-      }
-      if (tid == 0) {
-        if (!all_done) sm.status |= kStatusCorrupt;
-        if (t < d.out_T) {
-          uint64_t* row = step_stats + (uint64_t)t * kStepStats;
-          row[8] = tw1 - sm.t_wait;
-          row[9] = wall_clock64() - tw1;
-        }
-      }
-      // the helpers' counters and the step's push counts, read together
-      const unsigned long long cw = waits ? ld_relaxed(&dones[2 * (tid + 1) + 1]) : 0ull;
-      const unsigned long long pw = ld_relaxed(&ctl->pushes);
-      sh_next = (uint32_t)pw;
-      sh_sel = (uint32_t)(pw >> 32);
-      const uint32_t wc = wave_sum((uint32_t)cw), wp = wave_sum((uint32_t)(cw >> 32));
-      if (tid == 0) {
-        sm.w_children = lead_ch;
-        sm.w_probes = lead_pr;
-      }
-      __syncthreads();
-      if ((tid & 63u) == 0u) {
-        if (wc) atomicAdd(&sm.w_children, wc);
-        if (wp) atomicAdd(&sm.w_probes, wp);
-      }
-      if (!kLean || sv.cut_mode != kCutAbove || sh_next >= beams[t] || !all_done) break;
-      // too few pushes reach the cut: the others, in a second round
-      sv.cut_mode = kCutBelow;
-      __syncthreads();
-      lead_ch = sm.w_children;
-      lead_pr = sm.w_probes;
-      n_stolen = 0;
-      stole = false;
-      __syncthreads();
-      if (tid == 0) {
-        sm.w_children = 0;
-        sm.w_probes = 0;
-        sm.lq_next = 0;
-        sm.lq_sel = 0;
       }
     }
     __syncthreads();
@@ -3014,10 +3325,16 @@ __global__ void __launch_bounds__(kBlock) tbs_kernel(KArgs a) {
     // 0 adds the overflow bit below, which every thread derives itself
     const bool overflow = n_next > next_cap || nS + n_new > sel_cap;
     const bool stop = overflow || sm.status != 0;
+    if constexpr (!kLean) n_cands += (uint64_t)n_next + n_new;
     if (tid == 0) {
-      lds_add(&sm.n_cands, (uint64_t)n_next + n_new);
-      lds_add(&sm.cnt_children, w_ch);
-      lds_add(&sm.cnt_probes, w_pr);
+      if constexpr (kLean) {
+        lds_add(&sm.n_cands, (uint64_t)n_next + n_new);
+        lds_add(&sm.cnt_children, w_ch);
+        lds_add(&sm.cnt_probes, w_pr);
+      } else {
+        sm.cnt_children += w_ch;
+        sm.cnt_probes += w_pr;
+      }
       if (overflow) sm.status |= kStatusOverflow;
     }
     if (stop) {
@@ -3025,7 +3342,8 @@ __global__ void __launch_bounds__(kBlock) tbs_kernel(KArgs a) {
       break;
     }
     const unsigned long long t1 = wall_clock64();
-    if (tid == 0) lds_add(&sm.t_exp, t1 - t0);
+    if constexpr (!kLean) t_exp += t1 - t0;
+    else if (tid == 0) lds_add(&sm.t_exp, t1 - t0);
     if (tid == 0 && t < d.out_T) {
       uint64_t* row = step_stats + (uint64_t)t * kStepStats;
       row[0] = ncur0;
@@ -3148,7 +3466,8 @@ __global__ void __launch_bounds__(kBlock) tbs_kernel(KArgs a) {
       }
     }
     if (stop_after) {
-      if (tid == 0) lds_add(&sm.t_sel, wall_clock64() - t1);
+      if constexpr (!kLean) t_sel += wall_clock64() - t1;
+      else if (tid == 0) lds_add(&sm.t_sel, wall_clock64() - t1);
       break;
     }
 
@@ -3248,10 +3567,10 @@ __global__ void __launch_bounds__(kBlock) tbs_kernel(KArgs a) {
           // a child of the root: its entry from the root directory
           const uint4* rp = (const uint4*)&a.root_dir[tk];
           const uint4 rx = rp[0], ry = rp[1];
-          if (rx.x == c.node && !(rx.y & kRdErr)) e = root_child_entry(a, rx, ry, K);
-          else e = parent_entry<kLouds>(a, c.node, t + 1, K, &err);
+          if (rx.x == c.node && !(rx.y & kRdErr)) e = root_child_entry<kLean>(a, rx, ry, K);
+          else e = parent_entry<kLouds, kLean>(a, c.node, t + 1, K, &err);
         } else {
-          e = parent_entry<kLouds>(a, c.node, t + 1, K, &err);
+          e = parent_entry<kLouds, kLean>(a, c.node, t + 1, K, &err);
         }
       }
       const double s2 = ps + (double)x;
@@ -3354,7 +3673,8 @@ __global__ void __launch_bounds__(kBlock) tbs_kernel(KArgs a) {
       cur_which ^= 1u;
     }
     par_ready = next_table;
-    if (tid == 0) lds_add(&sm.t_sel, wall_clock64() - t1);
+    if constexpr (!kLean) t_sel += wall_clock64() - t1;
+    else if (tid == 0) lds_add(&sm.t_sel, wall_clock64() - t1);
   }
   // release the helpers
   if (tid == 0) st_dev(&ctl->go, tag | kGoExit);
@@ -3471,10 +3791,16 @@ __global__ void __launch_bounds__(kBlock) tbs_kernel(KArgs a) {
   if (tid == 0) {
     oh->count = status ? 0 : nS;
     const unsigned long long tend = wall_clock64();
-    oh->ticks_expand = sm.t_exp;
-    oh->ticks_select = sm.t_sel;
-    oh->ticks_total = tend - sm.t_all0;
-    oh->candidates = sm.n_cands;
+    if constexpr (kLean) {
+      t_exp = sm.t_exp;
+      t_sel = sm.t_sel;
+      t_all0 = sm.t_all0;
+      n_cands = sm.n_cands;
+    }
+    oh->ticks_expand = t_exp;
+    oh->ticks_select = t_sel;
+    oh->ticks_total = tend - t_all0;
+    oh->candidates = n_cands;
     oh->parents = sm.cnt_parents;
     oh->children = sm.cnt_children;
     oh->probes = sm.cnt_probes;
@@ -3587,7 +3913,7 @@ __global__ void __launch_bounds__(256) root_dir_kernel(KArgs a, RootEnt* dir, ui
   const ft_node_rec r = a.recs[ch];
   if (r.first_tok >= root_n) return;  // (the host sized the directory on these tokens)
   uint32_t err = 0;
-  const ParEntry e = parent_entry<false>(a, ch, 1u, 1u, &err);
+  const ParEntry e = parent_entry<false, true>(a, ch, 1u, 1u, &err);
   const uint32_t sd = r.meta & FT_META_DEPTH_MASK;
   const uint32_t el = (r.meta >> FT_META_ELEN_SHIFT) & FT_META_ELEN_MASK;
   const bool link = (r.meta & FT_META_TERMINAL) && sd > 1u;

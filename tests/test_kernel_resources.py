@@ -43,3 +43,10 @@ def test_no_scratch(kernels, streamed, lean):
     assert k[".private_segment_fixed_size"] == 0, k
     assert k[".vgpr_spill_count"] == 0, k
     assert not k.get(".uses_dynamic_stack", False), k
+
+
+@pytest.mark.parametrize("streamed", [0, 1])
+def test_general_holds_nothing_of_the_lean_one(kernels, streamed):
+    """The row's token bits (4 KB) are the lean instantiation's alone."""
+    general, lean = (kernels[0, streamed, x][".group_segment_fixed_size"] for x in (0, 1))
+    assert general + 4096 <= lean <= 160 * 1024
