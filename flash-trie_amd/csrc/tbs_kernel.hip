@@ -68,11 +68,9 @@ constexpr uint32_t kRowHashEmpty = 0xFFFFFFFFu;
 // a label whose bit is clear is not in the row
 constexpr int kRowBitsLog2 = 15;
 constexpr uint32_t kRowBits = 1u << kRowBitsLog2;
-// expansion: chunks of work items whose filter words a wave reads at once,
-// and the items it holds that passed the filters (at most 63 left over and
-// those of these chunks)
-constexpr uint32_t kQueueChunks = 1;
-constexpr uint32_t kQueueCap = 64u * (kQueueChunks + 1u);
+// expansion: the items a wave holds that passed the filters (at most 63 left
+// over and those of one chunk)
+constexpr uint32_t kQueueCap = 128;
 // the leader hashes the row for steps of at least this many work items (a
 // smaller step does too few lookups to repay the build)
 constexpr uint32_t kRowHashMinWork = 2048;
@@ -1585,80 +1583,69 @@ __device__ __forceinline__ void expand_lean(const KArgs& a, const StepView& v, u
     bool matched = false;  // (queued) its first fingerprint word matched
     if (queued) {
       while (n_q < 64u && c < nchunks) {
-        // what each item is (pk) and the word its filter looks at (every lane
-        // reads, an item without a filter the first label, so that the reads
-        // of all the chunks go out before the first is waited for)
-        uint32_t pk[kQueueChunks];
-        uint64_t pw[kQueueChunks];
-#pragma unroll
-        for (uint32_t u = 0; u < kQueueChunks; ++u) {
-          pk[u] = kPkNone;
-          const uint64_t* at = (const uint64_t*)labels;
-          const uint32_t w = (c << 6) + lane;
-          if (c < nchunks) {
-            // the chunk's parents: at or after the last chunk's, in one round
-            // of the search above when they are among the next 64
-            const uint32_t w0 = c << 6, wl = min(w0 + 63u, W - 1u);
-            const uint32_t o = sm.woff[min(p_at + lane, v.n_par)];
-            const uint64_t m0 = __ballot(o <= w0), m1 = __ballot(o <= wl);
-            uint32_t pa = p_at + (63u - (uint32_t)__clzll((long long)m0));
-            uint32_t pb = p_at + (64u - (uint32_t)__clzll((long long)m1));
-            if (m1 == ~0ull) chunk_parents(c, pa, pb);
-            p_at = pa;
-            if (w < W) {
-              uint32_t lo = pa, hi = pb;
-              while (hi - lo > 1) {
-                const uint32_t mid = (lo + hi) >> 1;
-                if (sm.woff[mid] <= w) lo = mid; else hi = mid;
-              }
-              const uint32_t i = w - sm.woff[lo], md = sm.p_mode[lo], c0 = sm.p_c0[lo];
-              const uint32_t item = (lo << 16) | i;
-              pk[u] = kPkAll | item;
-              if ((md & kModeMask) == M_SCAN) {
-                const uint32_t n = c0 + i;
-                ++my_children;
-                pk[u] = kPkScan | item | ((n & 1u) ? kPkBit : 0u);
-                at = (const uint64_t*)(labels + (n & ~1u));
-              } else if ((md & kModeMask) == M_HASH) {
-                const double x = (double)sm.row_lp[i], s = sm.p_s[lo] + x;
-                bool low = x <= (double)v.tok_thr || s <= v.sent_thr;
-                // a proposal on the round's other side of the cut is not
-                // looked up where its child could only go to `next`
-                if (v.cut_mode != kCutNone && ((md & kModeOpen) || !(md & kModeDepthOk) ||
-                                               v.cut_mode == kCutBelow))
-                  low = low || (s * v.lnf_next >= v.cut) != (v.cut_mode == kCutAbove);
-                if (low) {
-                  pk[u] = kPkNone;
-                } else if (md & kModeFiltered) {
-                  pk[u] = kPkHash | item;
-                  at = wfp + (c0 + cuckoo_h1(sm.row_id[i], sm.p_aux[lo]));
-                }
-              }
+        // what each item is (e) and the word its filter looks at (every lane
+        // reads, an item without a filter the first label: one read a chunk,
+        // without a branch around it)
+        uint32_t e = kPkNone;
+        const uint64_t* at = (const uint64_t*)labels;
+        const uint32_t w = (c << 6) + lane;
+        // the chunk's parents: at or after the last chunk's, in one round of
+        // the search above when they are among the next 64
+        const uint32_t w0 = c << 6, wl = min(w0 + 63u, W - 1u);
+        const uint32_t o = sm.woff[min(p_at + lane, v.n_par)];
+        const uint64_t m0 = __ballot(o <= w0), m1 = __ballot(o <= wl);
+        uint32_t pa = p_at + (63u - (uint32_t)__clzll((long long)m0));
+        uint32_t pb = p_at + (64u - (uint32_t)__clzll((long long)m1));
+        if (m1 == ~0ull) chunk_parents(c, pa, pb);
+        p_at = pa;
+        if (w < W) {
+          uint32_t lo = pa, hi = pb;
+          while (hi - lo > 1) {
+            const uint32_t mid = (lo + hi) >> 1;
+            if (sm.woff[mid] <= w) lo = mid; else hi = mid;
+          }
+          const uint32_t i = w - sm.woff[lo], md = sm.p_mode[lo], c0 = sm.p_c0[lo];
+          const uint32_t item = (lo << 16) | i;
+          e = kPkAll | item;
+          if ((md & kModeMask) == M_SCAN) {
+            const uint32_t n = c0 + i;
+            ++my_children;
+            e = kPkScan | item | ((n & 1u) ? kPkBit : 0u);
+            at = (const uint64_t*)(labels + (n & ~1u));
+          } else if ((md & kModeMask) == M_HASH) {
+            const double x = (double)sm.row_lp[i], s = sm.p_s[lo] + x;
+            bool low = x <= (double)v.tok_thr || s <= v.sent_thr;
+            // a proposal on the round's other side of the cut is not looked
+            // up where its child could only go to `next`
+            if (v.cut_mode != kCutNone && ((md & kModeOpen) || !(md & kModeDepthOk) ||
+                                           v.cut_mode == kCutBelow))
+              low = low || (s * v.lnf_next >= v.cut) != (v.cut_mode == kCutAbove);
+            if (low) {
+              e = kPkNone;
+            } else if (md & kModeFiltered) {
+              e = kPkHash | item;
+              at = wfp + (c0 + cuckoo_h1(sm.row_id[i], sm.p_aux[lo]));
             }
           }
-          c += nwaves;
-          pw[u] = *at;
         }
-#pragma unroll
-        for (uint32_t u = 0; u < kQueueChunks; ++u) {
-          const uint32_t kind = pk[u] & kPkNone;
-          const uint32_t w0 = (uint32_t)pw[u], w1 = (uint32_t)(pw[u] >> 32);
-          bool want = kind == kPkAll;
-          uint32_t e = pk[u];
-          if (kind == kPkScan) {
-            const uint32_t bit = row_bit(((e & kPkBit) ? w1 : w0) & kTokMask);
-            want = (sm.rh_bits[bit >> 5] >> (bit & 31u)) & 1u;
-          } else if (kind == kPkHash) {
-            const uint32_t f4 = wide_fp(sm.row_id[e & 0xFFFFu]) * 0x01010101u;
-            const bool first = has_zero_byte(w0 ^ f4) || has_zero_byte(w1 ^ f4);
-            // (a full first bucket without a match: the second may hold it)
-            want = first || !(has_zero_byte(w0) || has_zero_byte(w1));
-            if (first) e |= kPkBit;
-          }
-          const uint64_t m = __ballot(want);
-          if (want) qd[n_q + lanemask_lt_count(m)] = e;
-          n_q += (uint32_t)__popcll(m);
+        c += nwaves;
+        const uint64_t word = *at;
+        const uint32_t lo4 = (uint32_t)word, hi4 = (uint32_t)(word >> 32);
+        const uint32_t kind = e & kPkNone;
+        bool want = kind == kPkAll;
+        if (kind == kPkScan) {
+          const uint32_t bit = row_bit(((e & kPkBit) ? hi4 : lo4) & kTokMask);
+          want = (sm.rh_bits[bit >> 5] >> (bit & 31u)) & 1u;
+        } else if (kind == kPkHash) {
+          const uint32_t f4 = wide_fp(sm.row_id[e & 0xFFFFu]) * 0x01010101u;
+          const bool first = has_zero_byte(lo4 ^ f4) || has_zero_byte(hi4 ^ f4);
+          // (a full first bucket without a match: the second may hold it)
+          want = first || !(has_zero_byte(lo4) || has_zero_byte(hi4));
+          if (first) e |= kPkBit;
         }
+        const uint64_t m = __ballot(want);
+        if (want) qd[n_q + lanemask_lt_count(m)] = e;
+        n_q += (uint32_t)__popcll(m);
       }
       if (n_q == 0) break;
       // (the queue is the wave's own: LDS runs a wave's accesses in order)
