@@ -1359,11 +1359,16 @@ static KArgs kernel_args(const ft_ctx* c, const uint8_t* stage, size_t first, si
   a.wgs = std::max(1u, std::min(std::min(c->wgs_req, fit), lay.claim_slots));
   a.share_min = c->share_min;
   a.cut_pairs = c->cut_pairs;
-  // the lean instantiation, where beams and rows fit it and the pairs of a step
-  // may be enough for its queue (at beam = K = 1000 from batch 2 on; on
-  // smaller batches and beams it gains nothing, and measured 0-2% slower)
+  // The lean instantiation, where beams and rows fit it and a step is likely
+  // to reach its queue: two thirds of the widest beam's (parent, proposal)
+  // pairs are more items than its line (over the 800M-key trie step 1 has 0.5
+  // to 0.7 items a pair; a parent that is scanned has at most its children).
+  // Without the queue it gains nothing: 128 staged requests of beam = K = 250
+  // in launches of 32 take 91.9 us of device time each with the general
+  // instantiation and 94.9 with this one (5.4 chunks a wave in step 1).
+  const uint32_t per = bmax >= kCutMinBeam ? kCutMinChunks : kQueueMinChunks;
   a.lean = c->lean && kmax <= kBlockThreads && bmax <= kBlockThreads &&
-                   bmax * kmax > (uint64_t)kQueueMinChunks * kBlockThreads * a.wgs
+                   2 * bmax * kmax > 3ull * per * kBlockThreads * a.wgs
                ? 1u
                : 0u;
   uint32_t ep = ++g_launch_epoch;

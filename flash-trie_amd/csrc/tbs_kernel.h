@@ -19,9 +19,11 @@ constexpr uint32_t kNoHist = 0xFFFFFFFFu;
 // Threads of the search kernel's workgroups: the longest beam and row of its
 // lean instantiation.
 constexpr uint32_t kBlockThreads = 1024;
-// A step is queued (queues_items) when its 64-item chunks are more than this
-// many for each wave of its workgroups.
-constexpr uint32_t kQueueMinChunks = 4;
+// A step of the lean instantiation is queued (see has_chunks) when it has more
+// 64-item chunks than kQueueMinChunks for each wave of its workgroups, and also,
+// for a beam of at least kCutMinBeam, when it has more than kCutMinChunks and a
+// cut is found.
+constexpr uint32_t kQueueMinChunks = 8, kCutMinChunks = 4, kCutMinBeam = 640;
 
 enum : uint32_t { kReqEarlyExit = 1u, kReqSkip = 2u };
 
@@ -269,8 +271,8 @@ struct Ctl {
   // streamed search: (launch epoch << 32) | 1 once the leader has copied
   // the request's first rows to the device stage
   unsigned long long head;
-  // the shared step's cut of its `next` pushes (see cut_of_step): the norm's
-  // order-preserving key, and which pushes the round takes (kCut*)
+  // the shared step's cut of its `next` pushes (see cut_of_step): the norm,
+  // and which pushes the round takes (kCut*, kStepQueued)
   unsigned long long cut;
   // streamed search: the copy of the rows after the first ready word's
   // (launch epoch << 32) | kCopy* state, claimed by helper 1 or the leader

@@ -1104,15 +1104,19 @@ struct StepView {
   uint32_t keep_lds_max;
   // every parent has exactly one work item (item w belongs to parent w)
   bool one_each;
-  // (queued) the round's cut of the `next` pushes
+  // (lean) whether the step's items are queued (queues_step), and then the
+  // round's cut of the `next` pushes
+  bool queued;
   double cut;
   uint32_t cut_mode;
 };
 
-// The cut of a shared step (cut_of_step).  kCutNone: every push.  kCutAbove:
+// The cut of a shared, queued step (cut_of_step).  kCutNone: every push.  kCutAbove:
 // the pushes into `next` whose norm is at least `cut`, and every one into
 // `selected`.  kCutBelow: the other pushes into `next`, none into `selected`.
 enum : uint32_t { kCutNone = 0u, kCutAbove = 1u, kCutBelow = 2u };
+// beside them in Ctl::cut_mode: the step's items are queued
+constexpr uint32_t kStepQueued = 4u;
 
 // Position of tok in a sorted row held in the device stage (a row longer
 // than the LDS row arrays), or -1.  Device-coherent loads: a streamed
@@ -1143,14 +1147,20 @@ static_assert(kBlock <= 1024, "a parent index of the LDS table has 10 bits");
 // runs the filters alone over its chunks, one 8-byte read an item, and queues
 // the survivors in LDS; the rest runs on 64 of them at a time.  Bound by the
 // device's rate of random lines from there: two or three chunks' reads in
-// flight a wave gained nothing.  Taken when a wave has more than four chunks
-// (beam = K = 1000, step 1 of 512K items over the 800M-key trie, without a cut:
-// 16 chunks a wave at batch 8, 54.5 -> 46.9 us; 126 at batch 64, 573 -> 510
-// us); with fewer there is nothing to gather, and the queue's own latency
-// shows (batch 1, two chunks: 19.0 -> 20.0 us).
-__device__ __forceinline__ bool queues_items(const KArgs& a, const StepView& v, uint32_t W,
-                                             uint32_t nwaves, bool hashed) {
-  return hashed && ((W + 63u) >> 6) > kQueueMinChunks * nwaves && a.scan_limit <= 65536u;
+// flight a wave gained nothing.
+//
+// Whether a step has more than `per` chunks for each of its waves.  A wave of
+// few chunks has nothing to gather, and the queue's own latency shows; step 1
+// over the 800M-key trie without a cut, by chunks a wave: 4.3 (beam = K = 700,
+// batch 4) 23.2 -> 26.0 us, 4.7 (500, batch 8) 23.2 -> 26.8, 5.5 (250, batch 32)
+// 26.2 -> 27.5, 8.4 (700, batch 8) 32.4 -> 32.3, 9.3 (500, batch 16) 34.9 -> 33.6,
+// 10.9 (250, batch 64) 57.3 -> 53.3, 16 (1000, batch 8) 54.5 -> 46.9, 126 (1000,
+// batch 64) 573 -> 510: kQueueMinChunks is 8.  With a cut, which needs the
+// queue, the selection after the step gains as well, in proportion to the beam
+// (700, batch 4: 17.9 -> 13.7 us; 500, batch 8: 16.0 -> 13.1): beams from
+// kCutMinBeam on take the two from kCutMinChunks on, where a cut is found.
+__device__ __forceinline__ bool has_chunks(uint32_t W, uint32_t nwaves, uint32_t per) {
+  return ((W + 63u) >> 6) > per * nwaves;
 }
 
 // Chooses the cut of a shared step whose items are queued.  Of the pushes into
@@ -1529,7 +1539,7 @@ __device__ __forceinline__ void expand_range(const KArgs& a, const StepView& v, 
 }
 
 // expand_range of the lean instantiation (see tbs_kernel): the parent table
-// and the row are in LDS, a step of many chunks is queued (queues_items), and
+// and the row are in LDS, a step of many chunks is queued (has_chunks), and
 // a round may have a cut.  A function of its own: with one text for both (the
 // items in a shared lambda or loop) the general instantiation's expansion was
 // slower in every step, 52.5 -> 54.2 us a request over 128 staged requests of
@@ -1538,7 +1548,7 @@ __device__ __forceinline__ void expand_lean(const KArgs& a, const StepView& v, u
                              uint32_t gwave0, uint32_t nwaves, bool leader, bool solo,
                              bool hashed, SmemLean& sm) {
   const uint32_t tid = threadIdx.x, lane = tid & 63u;
-  const bool queued = queues_items(a, v, W, nwaves, hashed);
+  const bool queued = v.queued;
   uint32_t my_children = 0, my_probes = 0;
   const uint32_t K = v.K, t = v.t;
   const uint32_t nchunks = (W + 63u) >> 6;
@@ -2187,9 +2197,11 @@ __device__ __forceinline__ void helper_loop(const KArgs& a, const DevReq& d, uin
     const uint32_t mine = sm.hstep[6];
     double cut = 0.0;
     uint32_t cut_mode = kCutNone;
+    bool queued = false;
     if constexpr (kLean) {
       cut = __longlong_as_double((long long)sm.hcut);
-      cut_mode = sm.hcut_mode;
+      cut_mode = sm.hcut_mode & ~kStepQueued;
+      queued = (sm.hcut_mode & kStepQueued) != 0;
     }
     __syncthreads();
     if ((v >> 32) != a.epoch || (uint32_t)v == kGoExit || v == seen) return;
@@ -2232,6 +2244,7 @@ __device__ __forceinline__ void helper_loop(const KArgs& a, const DevReq& d, uin
     sv.sent_thr = d.sent_thr;
     sv.keep_lds_max = 0;
     sv.one_each = false;
+    sv.queued = queued;
     sv.cut = cut;
     sv.cut_mode = cut_mode;
     // the step's row (into the row hash too: emptied after the previous
@@ -2999,6 +3012,7 @@ __global__ void __launch_bounds__(kBlock) tbs_kernel(KArgs a) {
 
 
     const bool shared = a.wgs > 1 && W >= a.share_min;
+    sv.queued = false;
     sv.cut = 0.0;
     sv.cut_mode = kCutNone;
     uint32_t sh_next = 0, sh_sel = 0;  // (shared) the pushes of the step
@@ -3141,8 +3155,16 @@ __global__ void __launch_bounds__(kBlock) tbs_kernel(KArgs a) {
       }
     } else {
       const bool hashed = W >= kRowHashMinWork;
-      if (shared && queues_items(a, sv, W, a.wgs * (uint32_t)kWaves, hashed))
-        cut_of_step(a, sv, beams[t], (const uint64_t*)(in + d.kb_off) + 2ull * t, sm);
+      const uint32_t step_waves = (shared ? a.wgs : 1u) * (uint32_t)kWaves;
+      // (an item's place among its parent's fits the queue's 16 bits)
+      if (hashed && a.scan_limit <= 65536u) {
+        sv.queued = has_chunks(W, step_waves, kQueueMinChunks);
+        if (shared && (sv.queued || (beams[t] >= kCutMinBeam &&
+                                     has_chunks(W, step_waves, kCutMinChunks)))) {
+          cut_of_step(a, sv, beams[t], (const uint64_t*)(in + d.kb_off) + 2ull * t, sm);
+          sv.queued = sv.queued || sv.cut_mode != kCutNone;
+        }
+      }
       // the leader's slice 0, then (shared) the slices it takes over: one call
       // of the inlined expansion for both, which keeps its code and registers
       // to one copy
@@ -3165,7 +3187,7 @@ __global__ void __launch_bounds__(kBlock) tbs_kernel(KArgs a) {
             st_dev(&ctl->cur_which, cur_which);
             st_dev(&ctl->hist_n, hist_used);
             st_dev(&ctl->cut, (unsigned long long)__double_as_longlong(sv.cut));
-            st_dev(&ctl->cut_mode, sv.cut_mode);
+            st_dev(&ctl->cut_mode, sv.cut_mode | (sv.queued ? kStepQueued : 0u));
           }
           wait_stores();  // the step's data is complete before `go` moves
           __syncthreads();
