@@ -1187,22 +1187,43 @@ __device__ __forceinline__ void cut_of_step(const KArgs& a, StepView& v, uint32_
   const uint64_t pairs = (uint64_t)v.n_par * v.K, want = (uint64_t)a.cut_pairs * M;
   const uint64_t klo = kbound[0], khi = kbound[1];
   if (want == 0 || 2 * want > pairs || klo >= khi) return;
+  constexpr uint32_t kSide = 64, kPer = kSide * kSide / kBlock;
   const uint32_t md = tid < v.n_par ? (uint32_t)sm.p_mode[tid] : 0u;
   const bool skips =
       (md & kModeMask) == M_HASH && ((md & kModeOpen) || !(md & kModeDepthOk));
-  if (tid < 16u) sm.hist[tid] = 0;
+  if (tid <= kSide) sm.hist[tid] = 0;  // (counts of the search below, and n_s)
   const uint32_t n_skips = (uint32_t)__syncthreads_count(skips);
   if ((uint64_t)n_skips * v.K < want) return;
-  constexpr uint32_t kSide = 64, kPer = kSide * kSide / kBlock;
-  const double ps = sm.p_s[((tid & 63u) * v.n_par) / kSide];
+  // The sampled parents: about 48 of them, at most kSide, those with the least
+  // hashes of their nodes.  Not places in the table, whose order changes from
+  // run to run (survivors are emitted as they come): the cut, and with it the
+  // counters of the step, would change with it.
+  const uint32_t h = tid < v.n_par ? sm.p_node[tid] * 0x9E3779B1u : ~0u;
+  uint32_t lim = v.n_par <= kSide ? ~0u : (uint32_t)((48ull << 32) / v.n_par);
+  uint32_t n_s;
+  bool mine;
+  for (;;) {
+    mine = tid < v.n_par && h <= lim;
+    n_s = (uint32_t)__syncthreads_count(mine);
+    if (n_s <= kSide || lim < kSide) break;
+    lim -= lim >> 2;
+  }
+  if (n_s == 0 || n_s > kSide) return;  // (never more: the nodes are distinct)
+  // their scores, in any order (the row hash is not in use yet)
+  if (mine)
+    sm.bin_key[atomicAdd(&sm.hist[kSide], 1u)] =
+        (uint64_t)__double_as_longlong(sm.p_s[tid]);
+  __syncthreads();
+  const bool sampled = (tid & 63u) < n_s;
+  const double ps = sampled ? __longlong_as_double((long long)sm.bin_key[tid & 63u]) : 0.0;
   double norm[kPer];
 #pragma unroll
   for (uint32_t u = 0; u < kPer; ++u) {
     const double x = (double)sm.row_lp[((tid >> 6) * kPer + u) * v.K / kSide];
-    const bool low = x <= (double)v.tok_thr || ps + x <= v.sent_thr;
+    const bool low = !sampled || x <= (double)v.tok_thr || ps + x <= v.sent_thr;
     norm[u] = low ? -__builtin_inf() : (ps + x) * v.lnf_next;
   }
-  const uint32_t goal = max(1u, (uint32_t)(want * (kSide * kSide) / pairs));
+  const uint32_t goal = max(1u, (uint32_t)(want * (n_s * kSide) / pairs));
   auto value = [](uint64_t k) {  // the norm of a key
     return __longlong_as_double((long long)((k >> 63) ? k & 0x7FFFFFFFFFFFFFFFull : ~k));
   };
@@ -1619,7 +1640,7 @@ __device__ __forceinline__ void expand_lean(const KArgs& a, const StepView& v, u
           e = kPkAll | item;
           if ((md & kModeMask) == M_SCAN) {
             const uint32_t n = c0 + i;
-            ++my_children;
+            if (v.cut_mode != kCutBelow) ++my_children;  // (once a step)
             e = kPkScan | item | ((n & 1u) ? kPkBit : 0u);
             at = (const uint64_t*)(labels + (n & ~1u));
           } else if ((md & kModeMask) == M_HASH) {
@@ -3286,8 +3307,9 @@ __global__ void __launch_bounds__(kBlock) tbs_kernel(KArgs a) {
           if (!all_done) sm.status |= kStatusCorrupt;
           if (t < d.out_T) {
             uint64_t* row = step_stats + (uint64_t)t * kStepStats;
-            row[8] = tw1 - sm.t_wait;
-            row[9] = wall_clock64() - tw1;
+            // (the sums of a step's rounds; the rows start at 0)
+            row[8] += tw1 - sm.t_wait;
+            row[9] += wall_clock64() - tw1;
           }
         }
         // the helpers' counters and the step's push counts, read together

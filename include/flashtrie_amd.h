@@ -125,10 +125,18 @@ typedef struct ft_result {
   uint64_t* step_stats;  /* optional [num_steps * FT_STEP_STATS]: per step
                             parents, work items, next pushes, selected
                             pushes, expansion and selection ticks (wall
-                            clock), child records scanned, binary-search
-                            probes, and for a step shared between
+                            clock), child records scanned, probes of the
+                            lookups, and for a step shared between
                             workgroups the leader's wait for the helpers'
-                            claims and for their slices (ticks) */
+                            claims and for their slices (ticks).  A large
+                            step may leave pushes out of `next` that cannot
+                            survive it (those below a score that as many
+                            others reach as the beam keeps), with the
+                            lookups that only they need: they are not
+                            counted.  Where too few reach that score, a
+                            second round makes them after all: the children
+                            scanned count once, the probes and waits of both
+                            rounds add up */
 } ft_result;
 
 #define FT_STEP_STATS 10
@@ -139,10 +147,12 @@ typedef struct ft_timing {
   double expand_ms;       /* summed per-request device phase time */
   double select_ms;
   double other_ms;
-  uint64_t candidates;    /* next + selected pushes, summed over requests */
+  uint64_t candidates;    /* next + selected pushes, summed over requests
+                             (of those counted in step_stats) */
   uint64_t parents;       /* parents expanded */
   uint64_t children;      /* child records read by the scan path */
-  uint64_t probes;        /* binary-search probes of the search path */
+  uint64_t probes;        /* probes of the lookups: steps of a binary search,
+                             table buckets, root directory entries */
 } ft_timing;
 
 typedef struct ft_ctx ft_ctx;
