@@ -22,8 +22,10 @@ constexpr uint32_t kBlockThreads = 1024;
 // A step of the lean instantiation is queued (see has_chunks) when it has more
 // 64-item chunks than kQueueMinChunks for each wave of its workgroups, and also,
 // for a beam of at least kCutMinBeam, when it has more than kCutMinChunks and a
-// cut is found.
+// cut is found (beyond kCutMaybeChunks also a cut that has to be tried first, see
+// cut_of_step).
 constexpr uint32_t kQueueMinChunks = 8, kCutMinChunks = 4, kCutMinBeam = 640;
+constexpr uint32_t kCutMaybeChunks = 12;
 
 enum : uint32_t { kReqEarlyExit = 1u, kReqSkip = 2u };
 

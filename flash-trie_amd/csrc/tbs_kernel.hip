@@ -195,6 +195,8 @@ using SmemOf = std::conditional_t<kLean, SmemLean, Smem>;
 constexpr int kRankChunk = 1024;
 static_assert(offsetof(Smem, row_id) % 16 == 0 && offsetof(Smem, row_lp) % 16 == 0,
               "rank scratch is read 16 bytes at a time");
+static_assert(offsetof(Smem, bin_idx) >= offsetof(Smem, whist) + sizeof(Smem::whist),
+              "cut_of_step uses both at once");
 static_assert(kRankChunk == kBlock, "a thread's own rank entry sits in its own chunk");
 static_assert(kRankChunk % 16 == 0, "rank chunks hold whole count_before rounds");
 
@@ -1175,13 +1177,28 @@ __device__ __forceinline__ bool has_chunks(uint32_t W, uint32_t nwaves, uint32_t
 // and the leader checks their number; should fewer than M come, a second round
 // takes the rest.  The cut is the quantile of the scores of 64 x 64 sampled
 // (parent, proposal) pairs that lets cut_pairs * M pairs through: with 160, a
-// hit rate of 1 / 160 fills the beam in the first round, and the steps measured
-// have 1 / 110 to 1 / 30 (at beam = K = 1000, 5.1K pushes come).  Taken when
-// that is at most half of the pairs, and when the proposals that it can skip
-// are as many as those it lets through.  Step 1 at beam = K = 1000 over the
-// 800M-key trie: expansion 46.9 -> 41.5 and selection 25.1 -> 17.4 us at batch
-// 8, 510 -> 380 and 27.6 -> 18.1 us at batch 64.
-__device__ __forceinline__ void cut_of_step(const KArgs& a, StepView& v, uint32_t M,
+// hit rate of 1 / 160 fills the beam in the first round.  Over the 800M-key trie
+// the rate is 1 / 30 (at beam = K = 1000, 5.1K pushes come); other cuts there,
+// batch 8: 40 181 -> 211 us a call (second rounds), 80 175, 240 and 320 190.
+//
+// Tried only where it can gain: the cut lets at most half of the pairs through,
+// and as many proposals can be skipped (n_skips: hashed parents whose children
+// close no key).  And only where it can be trusted, because a second round costs
+// more than a cut gains: over 40M and 100M keys of the same vocabulary, beam = K
+// = 1000, where 0.9K to 1.1K pushes reach the cut, batch 8 took 187 us a call
+// without cuts and 211 with them, and 177 and 195.  The share of parents that are
+// hashed (so have many children) tells such tries from others: 0.20 and 0.26
+// there, 0.28 over 200M keys (2.2K pushes), 0.37 to 0.46 over the 800M (5.1 to
+// 7.2 pushes a kept hypothesis).  From 0.34 on the cut is taken as it is; below
+// that, sampled pairs are looked up first, 3 us, and only in steps of more than
+// kCutMaybeChunks chunks a wave, which can bear it (long keys, batch 8: 263 ->
+// 253 us; the 40M and 100M keys take 189 and 183).
+//
+// Step 1 at beam = K = 1000 over the 800M-key trie: expansion 46.9 -> 40.0 and
+// selection 25.1 -> 15.6 us at batch 8, 510 -> 355 and 27.6 -> 18.1 us at batch
+// 64.
+__device__ __forceinline__ void cut_of_step(const KArgs& a, StepView& v, uint32_t W,
+                                            uint32_t nwaves, uint32_t M,
                                             const uint64_t* kbound, Smem& sm) {
   const uint32_t tid = thread_idx<true>();
   const uint64_t pairs = (uint64_t)v.n_par * v.K, want = (uint64_t)a.cut_pairs * M;
@@ -1191,9 +1208,12 @@ __device__ __forceinline__ void cut_of_step(const KArgs& a, StepView& v, uint32_
   const uint32_t md = tid < v.n_par ? (uint32_t)sm.p_mode[tid] : 0u;
   const bool skips =
       (md & kModeMask) == M_HASH && ((md & kModeOpen) || !(md & kModeDepthOk));
-  if (tid <= kSide) sm.hist[tid] = 0;  // (counts of the search below, and n_s)
+  sm.whist[tid] = 0;
+  if (tid < 2u) sm.hist[tid] = 0;
   const uint32_t n_skips = (uint32_t)__syncthreads_count(skips);
   if ((uint64_t)n_skips * v.K < want) return;
+  const bool sure = n_skips * 50u >= v.n_par * 17u;
+  if (!sure && !has_chunks(W, nwaves, kCutMaybeChunks)) return;
   // The sampled parents: about 48 of them, at most kSide, those with the least
   // hashes of their nodes.  Not places in the table, whose order changes from
   // run to run (survivors are emitted as they come): the cut, and with it the
@@ -1209,13 +1229,12 @@ __device__ __forceinline__ void cut_of_step(const KArgs& a, StepView& v, uint32_
     lim -= lim >> 2;
   }
   if (n_s == 0 || n_s > kSide) return;  // (never more: the nodes are distinct)
-  // their scores, in any order (the row hash is not in use yet)
-  if (mine)
-    sm.bin_key[atomicAdd(&sm.hist[kSide], 1u)] =
-        (uint64_t)__double_as_longlong(sm.p_s[tid]);
+  // in any order (the row hash is not in use yet)
+  if (mine) sm.bin_idx[atomicAdd(&sm.hist[0], 1u)] = tid;
   __syncthreads();
   const bool sampled = (tid & 63u) < n_s;
-  const double ps = sampled ? __longlong_as_double((long long)sm.bin_key[tid & 63u]) : 0.0;
+  const uint32_t j = sampled ? sm.bin_idx[tid & 63u] : 0u;
+  const double ps = sm.p_s[j];
   double norm[kPer];
 #pragma unroll
   for (uint32_t u = 0; u < kPer; ++u) {
@@ -1227,23 +1246,58 @@ __device__ __forceinline__ void cut_of_step(const KArgs& a, StepView& v, uint32_
   auto value = [](uint64_t k) {  // the norm of a key
     return __longlong_as_double((long long)((k >> 63) ? k & 0x7FFFFFFFFFFFFFFFull : ~k));
   };
-  // the staged bounds hold every norm; 12 halvings of their range
-  double lo = value(klo), hi = value(khi);
-  bool found = false;
-#pragma unroll 1
-  for (uint32_t it = 0; it < 12u; ++it) {
-    const double mid = lo + 0.5 * (hi - lo);
-    uint32_t n = 0;
+  // The staged bounds hold every norm: a histogram over their range, one bin a
+  // thread, summed from its upper end.  (12 halvings of the range, a barrier
+  // and a count each, took 3 us more.)
+  const double lo = value(klo), range = value(khi) - lo;
+  if (!(range > 0.0 && range < 1e300)) return;
+  const double scale = (double)kBlock / range;
 #pragma unroll
-    for (uint32_t u = 0; u < kPer; ++u) n += (uint32_t)__popcll(__ballot(norm[u] >= mid));
-    if ((tid & 63u) == 0u) atomicAdd(&sm.hist[it], n);
+  for (uint32_t u = 0; u < kPer; ++u)
+    if (norm[u] >= lo)
+      atomicAdd(&sm.whist[min((uint32_t)((norm[u] - lo) * scale), (uint32_t)kBlock - 1u)], 1u);
+  __syncthreads();
+  const uint32_t bin = (uint32_t)kBlock - 1u - tid, count = sm.whist[bin];
+  uint32_t total;
+  const uint32_t above = block_excl_scan(count, &total, sm);
+  if (total < goal) return;
+  if (above < goal && above + count >= goal) sm.sel_digit = bin;
+  __syncthreads();
+  const double cut = lo + (double)sm.sel_digit / scale;
+  if (!sure) {
+    // Are there enough children behind them?  The sampled pairs from the cut up
+    // whose parent is hashed are looked up (first buckets only): M / pairs of the
+    // sample are M pushes; half as many again are asked for.
+    uint32_t n_hits = 0;
+    const bool looks = sampled && (sm.p_mode[j] & kModeMask) == M_HASH;
+    const uint32_t c0 = sm.p_c0[j], lg = sm.p_aux[j];
+    uint4 slots[kPer][2];
+#pragma unroll
+    for (uint32_t u = 0; u < kPer; ++u) {
+      const uint32_t tok = sm.row_id[((tid >> 6) * kPer + u) * v.K / kSide];
+      slots[u][0] = slots[u][1] =
+          make_uint4(kSlotEmptyTok, kSlotEmptyTok, kSlotEmptyTok, kSlotEmptyTok);
+      if (looks && norm[u] >= cut) {
+        const uint4* bw = (const uint4*)&a.wtab[c0 + cuckoo_h1(tok, lg)];
+        slots[u][0] = bw[0];
+        slots[u][1] = bw[1];
+      }
+    }
+#pragma unroll
+    for (uint32_t u = 0; u < kPer; ++u) {
+      const uint32_t tok = sm.row_id[((tid >> 6) * kPer + u) * v.K / kSide];
+      const uint4 x = slots[u][0], y = slots[u][1];
+      const bool hit = (x.x & kTokMask) == tok || (x.y & kTokMask) == tok ||
+                       (x.z & kTokMask) == tok || (x.w & kTokMask) == tok ||
+                       (y.x & kTokMask) == tok || (y.y & kTokMask) == tok ||
+                       (y.z & kTokMask) == tok || (y.w & kTokMask) == tok;
+      n_hits += (uint32_t)__popcll(__ballot(hit));
+    }
+    if ((tid & 63u) == 0u) atomicAdd(&sm.hist[1], n_hits);
     __syncthreads();
-    const bool enough = sm.hist[it] >= goal;
-    found = found || enough;
-    if (enough) lo = mid; else hi = mid;
+    if (2ull * sm.hist[1] * pairs < 3ull * M * (n_s * kSide)) return;
   }
-  if (!found) return;
-  v.cut = lo;
+  v.cut = cut;
   v.cut_mode = kCutAbove;
 }
 
@@ -3182,7 +3236,7 @@ __global__ void __launch_bounds__(kBlock) tbs_kernel(KArgs a) {
         sv.queued = has_chunks(W, step_waves, kQueueMinChunks);
         if (shared && (sv.queued || (beams[t] >= kCutMinBeam &&
                                      has_chunks(W, step_waves, kCutMinChunks)))) {
-          cut_of_step(a, sv, beams[t], (const uint64_t*)(in + d.kb_off) + 2ull * t, sm);
+          cut_of_step(a, sv, W, step_waves, beams[t], (const uint64_t*)(in + d.kb_off) + 2ull * t, sm);
           sv.queued = sv.queued || sv.cut_mode != kCutNone;
         }
       }
@@ -3637,7 +3691,7 @@ __global__ void __launch_bounds__(kBlock) tbs_kernel(KArgs a) {
       // only for a key on the boundary of a cut tie)
       if (tid == 0) sm.n_keep = n_listed;
       __syncthreads();
-      for (uint32_t b = tid; b < n_bin + ((kBlock - n_bin % kBlock) % kBlock); b += kBlock) {
+      for (uint32_t b = thread_idx<kLean>(); b < n_bin + ((kBlock - n_bin % kBlock) % kBlock); b += kBlock) {
         bool keep = false;
         uint32_t i = 0;
         if (b < n_bin) {
