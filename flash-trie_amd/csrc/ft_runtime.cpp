@@ -128,7 +128,8 @@ struct ft_ctx {
   uint32_t wgs_req = 4096;    // workgroups per request (clamped to residency:
                               // a lone request gets every CU)
   uint32_t share_min = 4096;  // work items from which a step is shared
-  uint64_t sort_min = 2048;   // proposals from which a batch is sorted on the device
+  uint64_t sort_min = 2048;   // proposals out of order that a batch needs to be
+                              // sorted on the device (see sorts_on_device)
   uint32_t cut_pairs = 160;   // see KArgs::cut_pairs
   bool lean = true;           // false: the general instantiation at any size
   // a streamed search publishes each request's first head_rows rows before
@@ -1664,30 +1665,44 @@ void pack_stream(PackJob& j, std::pair<uint32_t, uint32_t>* tmp) {
 }  // namespace
 
 namespace {
-// Whether a batch's rows are sorted on the device: some request's first row
-// is out of token order within its first kSortLook proposals, and every row
-// fits the sort.  A few compares a request decide, because the launch of a
-// batch in order waits for them (all of the first rows took 33 us of a batch
-// of 64): rows that come by score are out of order within the first few
-// proposals.  A batch whose disorder starts later is sorted on the packing
-// thread.  Against that sort (19 us a row of 777) the device pays one launch,
-// ~10 us, at any number of rows: calls with 2048 proposals in all take 107 us
-// with the thread's sort and 101 with the device's (rows of 256), with 1536
-// 104 and 110 (rows of 128); sort_min is the least that the device takes.
+// Whether a batch's rows are sorted on the device, looking at the first
+// kSortLook proposals of each request's first row (a few compares, because the
+// launch of a batch in order waits for them -- all of the first rows took 33 us
+// of a batch of 64 -- and rows that come by score are out of order within the
+// first few).  A batch whose disorder starts later is sorted on the packing
+// thread, and so is one with a row longer than the sort's.
+//
+// The packing thread's sort takes 10 to 20 ns a proposal of the requests out of
+// order (19 us a row of 777), the device's next to nothing, but a batch that
+// takes it is packed whole before anything is launched, its ordered requests
+// too: ~10 us for the launch, and what the overlap had hidden.  So the proposals
+// out of order are weighed against a constant, sort_min, and the ordered rest:
+// calls with 2048 proposals in all, shuffled, take 107 us with the thread's sort
+// and 101 with the device's, with 1536 104 and 110; batches of 64 with rows of
+// 100, of which 1, 4 and 32 requests (1200 proposals each) are out of order, 148,
+// 180 and 782 us with the thread's sort and 171 with the device's; with rows of
+// 32 and 1, 4 and 32 of them (384 each) 109, 114 and 250, and 132; with rows of
+// 500 and 1 and 4 of them (6000 each) 346 and 765, and 350.
 constexpr uint32_t kSortLook = 32;
 bool sorts_on_device(const ft_request* reqs, size_t batch, const StagedReq* staged,
                      uint64_t sort_min) {
-  bool raw = false;
-  uint64_t proposals = 0;
+  uint64_t unordered = 0, ordered = 0, ordered_reqs = 0;
   for (size_t r = 0; r < batch; ++r) {
     if (staged[r].skip) continue;
     const uint32_t K = staged[r].K;
     if (K > kMaxLdsTopk) return false;
-    proposals += (uint64_t)staged[r].T * K;
     const uint32_t* id = reqs[r].topk_id_rows ? reqs[r].topk_id_rows[0] : reqs[r].topk_id;
-    for (uint32_t k = 1; id && !raw && k < std::min(K, kSortLook); ++k) raw = id[k] <= id[k - 1];
+    bool out = false;
+    for (uint32_t k = 1; id && !out && k < std::min(K, kSortLook); ++k) out = id[k] <= id[k - 1];
+    if (out) {
+      unordered += (uint64_t)staged[r].T * K;
+    } else {
+      ordered += (uint64_t)staged[r].T * K;
+      ++ordered_reqs;
+    }
   }
-  return raw && proposals >= sort_min;
+  if (unordered == 0) return false;
+  return sort_min == 0 || unordered >= sort_min + 16 * ordered_reqs + ordered / 64;
 }
 
 // Packs every request of `j` with its rows as they came, and writes its ready

@@ -2,9 +2,12 @@
 against the CPU oracle, bit for bit (ranks of the caller's proposals break
 the ties that quantised logps make)."""
 
+import ctypes
+
 import numpy as np
 import pytest
 
+from cabi import Batch, check, load
 from helpers import assert_same_results
 
 pytestmark = pytest.mark.gpu
@@ -80,3 +83,44 @@ def test_bad_rows_are_refused(ft, trie, K):
     got = ft.bs_tbs_gpu(t, 3, beams, ids, lp, *args)  # and the context goes on
     for r in range(3):
         assert_same_results((got[0][r], got[1][r]), o.tbs([20] * 4, ids[r], lp[r], *args))
+
+
+# Which batches are sorted on the device: those with enough proposals out of
+# order for their ordered rest.  Every other is launched before its rows are
+# packed, so that a pause of the packing thread is part of the kernel's time.
+@pytest.mark.parametrize("B,K,n_out,device",
+                         [(16, 300, 0, False), (16, 300, 1, False), (16, 300, 2, False),
+                          (16, 300, 3, True), (16, 300, 16, True),
+                          (1, 511, 1, False), (1, 512, 1, True),
+                          (3, 4096, 1, True), (3, 4097, 3, False)])
+def test_which_batches(ft, po, monkeypatch, B, K, n_out, device):
+    monkeypatch.setenv("FT_PACK_DELAY_US", "20000")
+    toks, offs = ft.synth_keys(30000, VOCAB, 2, 5, 0.6, 3)
+    t = ft.Trie()
+    t.build_arrays(toks, offs)
+    image = np.array(t.image(), dtype=np.uint8)
+    o = po.OracleTrie.from_keys(toks=toks, offs=offs)
+    rng = np.random.default_rng(K + n_out)
+    ids, lp = _rows(rng, B, 4, K, VOCAB)
+    at = set(range(0, B, max(1, B // max(1, n_out)))[:n_out])
+    for r in range(B):
+        if r not in at:
+            ids[r].sort(axis=1)
+        else:
+            ids[r, 0, :2] = np.sort(ids[r, 0, :2])[::-1]
+    beams = np.full((B, 4), 20, dtype=np.uint32)
+    lib = load()
+    ctx = ctypes.c_void_p()
+    check(lib, lib.ft_create(image.ctypes.data, image.nbytes, 0, ctypes.byref(ctx)))
+    try:
+        check(lib, lib.ft_reserve(ctx, B, K, 4, 20, 80, 4096))
+        batch = Batch(beams, ids, lp, -4.0, -40.0, 5.0, False, 20)
+        timing = (ctypes.c_double * 8)()
+        print("B", B, "K", K, "out of order", n_out, flush=True)
+        check(lib, lib.ft_search(ctx, batch.reqs, B, batch.res, ctypes.byref(timing)))
+        assert (timing[0] < 15.0) == device, timing[0]
+        for r in range(B):
+            assert_same_results(batch.results(r), o.tbs(list(beams[r]), ids[r], lp[r], -4.0, -40.0,
+                                                        5.0, False), f"request {r}")
+    finally:
+        lib.ft_destroy(ctx)
