@@ -139,6 +139,7 @@ struct ft_ctx {
   // test knob: helpers never claim their slices, so the leader takes every
   // one over after its grace period
   uint32_t no_claims = 0;
+  uint32_t step_kinds = 0;    // see KArgs::step_kinds
   // a streamed search's bounded wait for a request's ready word (ticks),
   // and a delay before the host packs (microseconds): test knobs that
   // make requests come back not ready, to be searched again staged
@@ -785,6 +786,7 @@ int ft_create(const void* image, size_t image_bytes, int device,
     if (v >= 0) c->sort_min = (uint64_t)v;
   }
   if (const char* s = std::getenv("FT_TEST_NO_CLAIMS")) c->no_claims = std::atoi(s) ? 1u : 0u;
+  if (const char* s = std::getenv("FT_TEST_STEP_KINDS")) c->step_kinds = std::atoi(s) ? 1u : 0u;
   if (const char* s = std::getenv("FT_SCAN_MULT")) {
     const long v = std::strtol(s, nullptr, 10);
     if (v >= 0 && v < 1000000) c->scan_mult = (uint32_t)v;
@@ -1382,6 +1384,7 @@ static KArgs kernel_args(const ft_ctx* c, const uint8_t* stage, size_t first, si
   a.wdir_log2 = c->wdir_log2;
   a.wide_min = c->wide_min;
   a.no_claims = c->no_claims;
+  a.step_kinds = c->step_kinds;
   a.head_rows = 0;
   a.louds_words = c->d_louds_words;
   a.louds_z = c->d_louds_z;

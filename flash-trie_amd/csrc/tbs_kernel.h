@@ -26,6 +26,8 @@ constexpr uint32_t kBlockThreads = 1024;
 // cut_of_step).
 constexpr uint32_t kQueueMinChunks = 8, kCutMinChunks = 4, kCutMinBeam = 640;
 constexpr uint32_t kCutMaybeChunks = 12;
+// KArgs::step_kinds: the step was queued, had a cut, took a second round.
+enum : uint32_t { kKindQueued = 1u, kKindCut = 2u, kKindTwice = 4u };
 
 enum : uint32_t { kReqEarlyExit = 1u, kReqSkip = 2u };
 
@@ -326,6 +328,9 @@ struct KArgs {
   // every beam width and K of the launch is at most the kernel's block and a
   // step may have enough items for its queue: the lean instantiation runs
   uint32_t lean;
+  // step_stats' last word says how the lean instantiation expanded the step
+  // (kKind*) in place of the wait (for tests; never set otherwise)
+  uint32_t step_kinds;
   // helpers never claim their slices (a test of the leader's take-over of
   // unclaimed slices; never set otherwise)
   uint32_t no_claims;

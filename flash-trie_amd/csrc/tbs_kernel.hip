@@ -3397,6 +3397,10 @@ __global__ void __launch_bounds__(kBlock) tbs_kernel(KArgs a) {
           sm.lq_sel = 0;
         }
       }
+      if (a.step_kinds && tid == 0 && t < d.out_T)
+        (step_stats + (uint64_t)t * kStepStats)[9] =
+            (sv.queued ? kKindQueued : 0u) | (sv.cut_mode != kCutNone ? kKindCut : 0u) |
+            (sv.cut_mode == kCutBelow ? kKindTwice : 0u);
     }
     __syncthreads();
     // the helpers' pushes are complete (they waited for their stores before

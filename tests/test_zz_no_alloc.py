@@ -88,6 +88,27 @@ def test_noalloc_shared_steps(ft, trie, monkeypatch):
         lib.ft_destroy(ctx)
 
 
+def test_noalloc_queued_steps(ft, trie, monkeypatch):
+    # the instantiation for large steps: two requests of two workgroups, every
+    # parent looked up (step 1 says that it was queued)
+    for k, v in dict(FT_WGS="2", FT_WIDE_MIN="2", FT_SCAN_MULT="0",
+                     FT_TEST_STEP_KINDS="1").items():
+        monkeypatch.setenv(k, v)
+    t, image, o = trie
+    lib = load()
+    ctx = _ctx(lib, image)
+    try:
+        check(lib, lib.ft_reserve(ctx, 2, 500, 8, 300, 300 * 8, 4096))
+        r1, n1, a1 = _batch(ft, t, 70, 2, 8, 500, 300, 38)
+        stats = np.zeros((2, 8, 10), dtype=np.uint64)
+        for i in range(2):
+            n1.res[i].step_stats = stats[i].ctypes.data_as(ctypes.POINTER(ctypes.c_uint64))
+        _same(lib, ctx, r1, n1, "queued steps, batch 2, beam 300, K 500", o, a1)
+        assert (stats[:, 1, 9] & np.uint64(1)).all(), stats[:, 1]
+    finally:
+        lib.ft_destroy(ctx)
+
+
 def test_noalloc_beam_1000_and_limits(ft, trie):
     t, image, o = trie
     lib = load()
