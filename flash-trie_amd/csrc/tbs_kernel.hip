@@ -176,6 +176,9 @@ struct alignas(16) Smem {
   // the end of its share of the step
   NextRec push_next[kPushCap];
   SelRec push_sel[kPushSelCap];
+  // thread 0's of the leader: its clocks and the candidates so far (here rather
+  // than in registers through the steps, but in the staged search: see kTight)
+  unsigned long long t_exp, t_sel, t_all0, t_post, t_wait, n_cands;
 };
 // What the lean instantiation (see tbs_kernel) holds besides, behind the
 // layout that both share.
@@ -185,9 +188,6 @@ struct alignas(16) SmemLean : Smem {
   // a helper's view of the posted step's cut
   unsigned long long hcut;
   uint32_t hcut_mode;
-  // thread 0's of the leader: its clocks and the candidates so far (here
-  // rather than in registers through the steps)
-  unsigned long long t_exp, t_sel, t_all0, t_post, t_wait, n_cands;
 };
 template <bool kLean>
 using SmemOf = std::conditional_t<kLean, SmemLean, Smem>;
@@ -2827,9 +2827,14 @@ __global__ void __launch_bounds__(kBlock) tbs_kernel(KArgs a) {
   uint32_t gen = 0;
   unsigned long long t_post = 0;  // (thread 0) wall clock of the last post
 
-  // (the lean instantiation's clocks and its candidates are in LDS)
+  // Instantiations whose registers are full keep thread 0's clocks and the
+  // candidates in LDS and form the addresses of loops where they are used
+  // (thread_idx).  In the streamed search that takes 95.2 -> 93.3 us of device
+  // time at beam 500, batch 1 over 10M keys; the staged one, with fewer live
+  // values, loses by it: 91.8 -> 95.3 us a request at beam 250, launches of 32.
+  constexpr bool kTight = kLean || kStreamed;
   unsigned long long t_exp = 0, t_sel = 0, t_all0 = wall_clock64();
-  if constexpr (kLean) {
+  if constexpr (kTight) {
     if (tid == 0) sm.t_all0 = t_all0;
   }
   // per-step profile rows after the output tokens: kStepStats u64 per step
@@ -2840,7 +2845,7 @@ __global__ void __launch_bounds__(kBlock) tbs_kernel(KArgs a) {
     sm.status = 0;
     sm.multi_item = 0;
     sm.cnt_parents = sm.cnt_children = sm.cnt_probes = 0;
-    if constexpr (kLean) sm.t_exp = sm.t_sel = sm.n_cands = 0;
+    if constexpr (kTight) sm.t_exp = sm.t_sel = sm.n_cands = 0;
   }
   uint32_t n_cur = 1, nS = 0, hist_used = 0;
   uint64_t n_cands = 0;
@@ -2923,7 +2928,7 @@ __global__ void __launch_bounds__(kBlock) tbs_kernel(KArgs a) {
           n_cur = sm.tiny_ncur;
           nS = sm.tiny_nS;
           hist_used = sm.tiny_hist;
-          if constexpr (kLean) {
+          if constexpr (kTight) {
             if (tid == 0) {
               lds_add(&sm.n_cands, sm.tiny_cands);
               lds_add(&sm.t_exp, sm.tiny_ticks);
@@ -2957,7 +2962,7 @@ __global__ void __launch_bounds__(kBlock) tbs_kernel(KArgs a) {
       }
     } else {
       if (kLean || K <= kMaxLdsTopk) {
-        load_row<kLean>(rid, rlp, t, K, sm);
+        load_row<kTight>(rid, rlp, t, K, sm);
       } else if (tid == 0) {
         // a row longer than the LDS row arrays is searched in the stage
         // (the parent phase ends synchronised: every thread sees these)
@@ -3034,7 +3039,7 @@ __global__ void __launch_bounds__(kBlock) tbs_kernel(KArgs a) {
       }
     } else {
       for (uint32_t cbase = 0; cbase < (kLean ? 1u : n_cur); cbase += kBlock) {
-        const uint32_t j = cbase + (kLean ? thread_idx<kLean>() : tid);
+        const uint32_t j = cbase + (kTight ? thread_idx<kTight>() : tid);
         const uint32_t work = j < n_cur ? parent_work(j) : 0u;
         uint32_t Wc;
         const uint32_t off = block_excl_scan(work, &Wc, sm);
@@ -3051,7 +3056,7 @@ __global__ void __launch_bounds__(kBlock) tbs_kernel(KArgs a) {
       }
     }
     if (tid == 0) {
-      if constexpr (kLean) lds_add(&sm.cnt_parents, n_cur);
+      if constexpr (kTight) lds_add(&sm.cnt_parents, n_cur);
       else sm.cnt_parents += n_cur;
       // this workgroup's expansion counters (expand_range of the leader
       // relies on them being zero)
@@ -3112,7 +3117,8 @@ __global__ void __launch_bounds__(kBlock) tbs_kernel(KArgs a) {
         ++gen;
         if (tid == 0) {
           st_dev(&ctl->go, tag | gen);
-          t_post = wall_clock64();
+          if constexpr (kTight) sm.t_post = wall_clock64();
+          else t_post = wall_clock64();
         }
       }
       // (the parent table ended synchronised: the row and the emptied hash are
@@ -3137,7 +3143,9 @@ __global__ void __launch_bounds__(kBlock) tbs_kernel(KArgs a) {
         // taken over here -- so the step never waits for a workgroup that is
         // not running.  Then every claimed slice is waited for: a helper that
         // claimed one is running and finishes it.
-        const unsigned long long tw0 = wall_clock64();
+        unsigned long long tw0 = 0;
+        if constexpr (!kTight) tw0 = wall_clock64();
+        else if (tid == 0) sm.t_wait = wall_clock64();
         const unsigned long long mygo = tag | gen;
         unsigned long long* claims = (unsigned long long*)(ws + a.lay.claims);
         const uint32_t nh = a.wgs - 1;  // helper slots 1 .. nh (nh < kBlock)
@@ -3149,6 +3157,7 @@ __global__ void __launch_bounds__(kBlock) tbs_kernel(KArgs a) {
             pending_any = false;
             break;
           }
+          if constexpr (kTight) t_post = sm.t_post;
           if (tid == 0) sm.lead_flag = (wall_clock64() - t_post > kGraceTicks) ? 1u : 0u;
           __syncthreads();
           const bool expired = sm.lead_flag != 0;
@@ -3208,6 +3217,7 @@ __global__ void __launch_bounds__(kBlock) tbs_kernel(KArgs a) {
           if (!all_done) sm.status |= kStatusCorrupt;
           if (t < d.out_T) {
             uint64_t* row = step_stats + (uint64_t)t * kStepStats;
+            if constexpr (kTight) tw0 = sm.t_wait;
             row[8] = tw1 - tw0;
             row[9] = wall_clock64() - tw1;
           }
@@ -3414,9 +3424,9 @@ __global__ void __launch_bounds__(kBlock) tbs_kernel(KArgs a) {
     // 0 adds the overflow bit below, which every thread derives itself
     const bool overflow = n_next > next_cap || nS + n_new > sel_cap;
     const bool stop = overflow || sm.status != 0;
-    if constexpr (!kLean) n_cands += (uint64_t)n_next + n_new;
+    if constexpr (!kTight) n_cands += (uint64_t)n_next + n_new;
     if (tid == 0) {
-      if constexpr (kLean) {
+      if constexpr (kTight) {
         lds_add(&sm.n_cands, (uint64_t)n_next + n_new);
         lds_add(&sm.cnt_children, w_ch);
         lds_add(&sm.cnt_probes, w_pr);
@@ -3431,7 +3441,7 @@ __global__ void __launch_bounds__(kBlock) tbs_kernel(KArgs a) {
       break;
     }
     const unsigned long long t1 = wall_clock64();
-    if constexpr (!kLean) t_exp += t1 - t0;
+    if constexpr (!kTight) t_exp += t1 - t0;
     else if (tid == 0) lds_add(&sm.t_exp, t1 - t0);
     if (tid == 0 && t < d.out_T) {
       uint64_t* row = step_stats + (uint64_t)t * kStepStats;
@@ -3518,7 +3528,7 @@ __global__ void __launch_bounds__(kBlock) tbs_kernel(KArgs a) {
           stop_after = true;
         }
       } else {
-        b = bounded_select<kLean>(nU, F, sel_key, sel_arr, sel_node, compute_ranks, sm);
+        b = bounded_select<kTight>(nU, F, sel_key, sel_arr, sel_node, compute_ranks, sm);
       }
       if (b.all && !early_cut) {
         // every push fits: the new items simply become old ones (no LDS
@@ -3555,7 +3565,7 @@ __global__ void __launch_bounds__(kBlock) tbs_kernel(KArgs a) {
       }
     }
     if (stop_after) {
-      if constexpr (!kLean) t_sel += wall_clock64() - t1;
+      if constexpr (!kTight) t_sel += wall_clock64() - t1;
       else if (tid == 0) lds_add(&sm.t_sel, wall_clock64() - t1);
       break;
     }
@@ -3570,7 +3580,7 @@ __global__ void __launch_bounds__(kBlock) tbs_kernel(KArgs a) {
     auto nn = [&](uint32_t i) { return nextc[i].node; };
     const bool collect = kLean || M <= (uint32_t)kKeepCap;
     const uint64_t nk_lo = kbound[0], nk_hi = kbound[1];
-    const Bound bn = bounded_select<kLean>(n_next, M, nk, na, nn, compute_ranks, sm,
+    const Bound bn = bounded_select<kTight>(n_next, M, nk, na, nn, compute_ranks, sm,
                                     nk_lo <= nk_hi, nk_lo, nk_hi, collect);
     // survivors already listed by the selection (keys above its boundary
     // bin), and the boundary bin's size
@@ -3695,7 +3705,7 @@ __global__ void __launch_bounds__(kBlock) tbs_kernel(KArgs a) {
       // only for a key on the boundary of a cut tie)
       if (tid == 0) sm.n_keep = n_listed;
       __syncthreads();
-      for (uint32_t b = thread_idx<kLean>(); b < n_bin + ((kBlock - n_bin % kBlock) % kBlock); b += kBlock) {
+      for (uint32_t b = thread_idx<kTight>(); b < n_bin + ((kBlock - n_bin % kBlock) % kBlock); b += kBlock) {
         bool keep = false;
         uint32_t i = 0;
         if (b < n_bin) {
@@ -3714,7 +3724,7 @@ __global__ void __launch_bounds__(kBlock) tbs_kernel(KArgs a) {
     } else if (kLean || keep_cnt <= (uint32_t)kKeepCap) {
       // positions of the survivors first (from the keys alone; the rest of
       // a record is read only for a key on the boundary of a cut tie)
-      visit_keys<kLean>(n_next, nk, [&](uint32_t i, bool ok, uint64_t key) {
+      visit_keys<kTight>(n_next, nk, [&](uint32_t i, bool ok, uint64_t key) {
         bool keep = false;
         if (ok) {
           if (bn.all || key > bn.vkey) keep = true;
@@ -3762,7 +3772,7 @@ __global__ void __launch_bounds__(kBlock) tbs_kernel(KArgs a) {
       cur_which ^= 1u;
     }
     par_ready = next_table;
-    if constexpr (!kLean) t_sel += wall_clock64() - t1;
+    if constexpr (!kTight) t_sel += wall_clock64() - t1;
     else if (tid == 0) lds_add(&sm.t_sel, wall_clock64() - t1);
   }
   // release the helpers
@@ -3880,7 +3890,7 @@ __global__ void __launch_bounds__(kBlock) tbs_kernel(KArgs a) {
   if (tid == 0) {
     oh->count = status ? 0 : nS;
     const unsigned long long tend = wall_clock64();
-    if constexpr (kLean) {
+    if constexpr (kTight) {
       t_exp = sm.t_exp;
       t_sel = sm.t_sel;
       t_all0 = sm.t_all0;
