@@ -1613,17 +1613,13 @@ __device__ __forceinline__ void expand_range(const KArgs& a, const StepView& v, 
   expand_end(v, my_children, my_probes, solo, sm);
 }
 
-// expand_range of the lean instantiation (see tbs_kernel): the parent table
-// and the row are in LDS, a step of many chunks is queued (has_chunks), and
-// a round may have a cut.  A function of its own: with one text for both (the
-// items in a shared lambda or loop) the general instantiation's expansion was
-// slower in every step, 52.5 -> 54.2 us a request over 128 staged requests of
-// beam 250.
-__device__ __forceinline__ void expand_lean(const KArgs& a, const StepView& v, uint32_t W,
+// expand_range for a step whose items are queued (see has_chunks; the lean
+// instantiation): the parent table and the row are in LDS, and a round may have
+// a cut.
+__device__ __forceinline__ void expand_queued(const KArgs& a, const StepView& v, uint32_t W,
                              uint32_t gwave0, uint32_t nwaves, bool leader, bool solo,
                              bool hashed, SmemLean& sm) {
   const uint32_t tid = threadIdx.x, lane = tid & 63u;
-  const bool queued = v.queued;
   uint32_t my_children = 0, my_probes = 0;
   const uint32_t K = v.K, t = v.t;
   const uint32_t nchunks = (W + 63u) >> 6;
@@ -1652,8 +1648,8 @@ __device__ __forceinline__ void expand_lean(const KArgs& a, const StepView& v, u
   uint32_t c = (uint32_t)__builtin_amdgcn_readfirstlane((int)(slice + nwg * (tid >> 6)));
   uint32_t n_q = 0;
   uint32_t* qd = sm.ex_queue[tid >> 6];
-  uint32_t p_at = 0;  // (queued) the first parent of the last chunk looked at
-  // (queued) the arrays the filters read, held: the kernel's arguments are
+  uint32_t p_at = 0;  // the first parent of the last chunk looked at
+  // the arrays the filters read, held: the kernel's arguments are
   // otherwise loaded again, and waited for, in every round
   const uint32_t* labels = a.labels;
   const uint64_t* wfp = a.wfp;
@@ -1663,110 +1659,86 @@ __device__ __forceinline__ void expand_lean(const KArgs& a, const StepView& v, u
     uint32_t cnode = 0, pj = 0, k = 0, tok = 0;
     double s2 = 0.0;
     // the item of this lane: its parent and its place among the parent's
-    bool item_ok;
     uint32_t q = 0;
-    bool matched = false;  // (queued) its first fingerprint word matched
-    if (queued) {
-      while (n_q < 64u && c < nchunks) {
-        // what each item is (e) and the word its filter looks at (every lane
-        // reads, an item without a filter the first label: one read a chunk,
-        // without a branch around it)
-        uint32_t e = kPkNone;
-        const uint64_t* at = (const uint64_t*)labels;
-        const uint32_t w = (c << 6) + lane;
-        // the chunk's parents: at or after the last chunk's, in one round of
-        // the search above when they are among the next 64
-        const uint32_t w0 = c << 6, wl = min(w0 + 63u, W - 1u);
-        const uint32_t o = sm.woff[min(p_at + lane, v.n_par)];
-        const uint64_t m0 = __ballot(o <= w0), m1 = __ballot(o <= wl);
-        uint32_t pa = p_at + (63u - (uint32_t)__clzll((long long)m0));
-        uint32_t pb = p_at + (64u - (uint32_t)__clzll((long long)m1));
-        if (m1 == ~0ull) chunk_parents(c, pa, pb);
-        p_at = pa;
-        if (w < W) {
-          uint32_t lo = pa, hi = pb;
-          while (hi - lo > 1) {
-            const uint32_t mid = (lo + hi) >> 1;
-            if (sm.woff[mid] <= w) lo = mid; else hi = mid;
-          }
-          const uint32_t i = w - sm.woff[lo], md = sm.p_mode[lo], c0 = sm.p_c0[lo];
-          const uint32_t item = (lo << 16) | i;
-          e = kPkAll | item;
-          if ((md & kModeMask) == M_SCAN) {
-            const uint32_t n = c0 + i;
-            if (v.cut_mode != kCutBelow) ++my_children;  // (once a step)
-            e = kPkScan | item | ((n & 1u) ? kPkBit : 0u);
-            at = (const uint64_t*)(labels + (n & ~1u));
-          } else if ((md & kModeMask) == M_HASH) {
-            const double x = (double)sm.row_lp[i], s = sm.p_s[lo] + x;
-            bool low = x <= (double)v.tok_thr || s <= v.sent_thr;
-            // a proposal on the round's other side of the cut is not looked
-            // up where its child could only go to `next`
-            if (v.cut_mode != kCutNone && ((md & kModeOpen) || !(md & kModeDepthOk) ||
-                                           v.cut_mode == kCutBelow))
-              low = low || (s * v.lnf_next >= v.cut) != (v.cut_mode == kCutAbove);
-            if (low) {
-              e = kPkNone;
-            } else if (md & kModeFiltered) {
-              e = kPkHash | item;
-              at = wfp + (c0 + cuckoo_h1(sm.row_id[i], sm.p_aux[lo]));
-            }
-          }
-        }
-        c += nwaves;
-        const uint64_t word = *at;
-        const uint32_t lo4 = (uint32_t)word, hi4 = (uint32_t)(word >> 32);
-        const uint32_t kind = e & kPkNone;
-        bool want = kind == kPkAll;
-        if (kind == kPkScan) {
-          const uint32_t bit = row_bit(((e & kPkBit) ? hi4 : lo4) & kTokMask);
-          want = (sm.rh_bits[bit >> 5] >> (bit & 31u)) & 1u;
-        } else if (kind == kPkHash) {
-          const uint32_t f4 = wide_fp(sm.row_id[e & 0xFFFFu]) * 0x01010101u;
-          const bool first = has_zero_byte(lo4 ^ f4) || has_zero_byte(hi4 ^ f4);
-          // (a full first bucket without a match: the second may hold it)
-          want = first || !(has_zero_byte(lo4) || has_zero_byte(hi4));
-          if (first) e |= kPkBit;
-        }
-        const uint64_t m = __ballot(want);
-        if (want) qd[n_q + lanemask_lt_count(m)] = e;
-        n_q += (uint32_t)__popcll(m);
-      }
-      if (n_q == 0) break;
-      // (the queue is the wave's own: LDS runs a wave's accesses in order)
-      __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
-      const uint32_t take = min(n_q, 64u);
-      n_q -= take;
-      item_ok = lane < take;
-      if (item_ok) {
-        const uint32_t e = qd[n_q + lane];
-        pj = (e & kPkItem) >> 16;
-        q = e & 0xFFFFu;
-        matched = (e & kPkBit) != 0;
-      }
-      __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
-    } else {
-      if (c >= nchunks) break;
+    bool matched = false;  // its first fingerprint word matched
+    while (n_q < 64u && c < nchunks) {
+      // what each item is (e) and the word its filter looks at (every lane
+      // reads, an item without a filter the first label: one read a chunk,
+      // without a branch around it)
+      uint32_t e = kPkNone;
+      const uint64_t* at = (const uint64_t*)labels;
       const uint32_t w = (c << 6) + lane;
-      uint32_t pa = 0, pb = v.n_par;
-      if (!v.one_each) chunk_parents(c, pa, pb);
-      c += nwaves;
-      item_ok = w < W;
-      if (item_ok) {
-        // parent of work item w: the last j with woff[j] <= w
+      // the chunk's parents: at or after the last chunk's, in one round of
+      // the search above when they are among the next 64
+      const uint32_t w0 = c << 6, wl = min(w0 + 63u, W - 1u);
+      const uint32_t o = sm.woff[min(p_at + lane, v.n_par)];
+      const uint64_t m0 = __ballot(o <= w0), m1 = __ballot(o <= wl);
+      uint32_t pa = p_at + (63u - (uint32_t)__clzll((long long)m0));
+      uint32_t pb = p_at + (64u - (uint32_t)__clzll((long long)m1));
+      if (m1 == ~0ull) chunk_parents(c, pa, pb);
+      p_at = pa;
+      if (w < W) {
         uint32_t lo = pa, hi = pb;
-        if (v.one_each) {
-          lo = w;
-        } else {
-          while (hi - lo > 1) {
-            const uint32_t mid = (lo + hi) >> 1;
-            if (sm.woff[mid] <= w) lo = mid; else hi = mid;
+        while (hi - lo > 1) {
+          const uint32_t mid = (lo + hi) >> 1;
+          if (sm.woff[mid] <= w) lo = mid; else hi = mid;
+        }
+        const uint32_t i = w - sm.woff[lo], md = sm.p_mode[lo], c0 = sm.p_c0[lo];
+        const uint32_t item = (lo << 16) | i;
+        e = kPkAll | item;
+        if ((md & kModeMask) == M_SCAN) {
+          const uint32_t n = c0 + i;
+          if (v.cut_mode != kCutBelow) ++my_children;  // (once a step)
+          e = kPkScan | item | ((n & 1u) ? kPkBit : 0u);
+          at = (const uint64_t*)(labels + (n & ~1u));
+        } else if ((md & kModeMask) == M_HASH) {
+          const double x = (double)sm.row_lp[i], s = sm.p_s[lo] + x;
+          bool low = x <= (double)v.tok_thr || s <= v.sent_thr;
+          // a proposal on the round's other side of the cut is not looked
+          // up where its child could only go to `next`
+          if (v.cut_mode != kCutNone && ((md & kModeOpen) || !(md & kModeDepthOk) ||
+                                         v.cut_mode == kCutBelow))
+            low = low || (s * v.lnf_next >= v.cut) != (v.cut_mode == kCutAbove);
+          if (low) {
+            e = kPkNone;
+          } else if (md & kModeFiltered) {
+            e = kPkHash | item;
+            at = wfp + (c0 + cuckoo_h1(sm.row_id[i], sm.p_aux[lo]));
           }
         }
-        pj = lo;
-        q = w - sm.woff[pj];
       }
+      c += nwaves;
+      const uint64_t word = *at;
+      const uint32_t lo4 = (uint32_t)word, hi4 = (uint32_t)(word >> 32);
+      const uint32_t kind = e & kPkNone;
+      bool want = kind == kPkAll;
+      if (kind == kPkScan) {
+        const uint32_t bit = row_bit(((e & kPkBit) ? hi4 : lo4) & kTokMask);
+        want = (sm.rh_bits[bit >> 5] >> (bit & 31u)) & 1u;
+      } else if (kind == kPkHash) {
+        const uint32_t f4 = wide_fp(sm.row_id[e & 0xFFFFu]) * 0x01010101u;
+        const bool first = has_zero_byte(lo4 ^ f4) || has_zero_byte(hi4 ^ f4);
+        // (a full first bucket without a match: the second may hold it)
+        want = first || !(has_zero_byte(lo4) || has_zero_byte(hi4));
+        if (first) e |= kPkBit;
+      }
+      const uint64_t m = __ballot(want);
+      if (want) qd[n_q + lanemask_lt_count(m)] = e;
+      n_q += (uint32_t)__popcll(m);
     }
+    if (n_q == 0) break;
+    // (the queue is the wave's own: LDS runs a wave's accesses in order)
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    const uint32_t take = min(n_q, 64u);
+    n_q -= take;
+    const bool item_ok = lane < take;
+    if (item_ok) {
+      const uint32_t e = qd[n_q + lane];
+      pj = (e & kPkItem) >> 16;
+      q = e & 0xFFFFu;
+      matched = (e & kPkBit) != 0;
+    }
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
     if (item_ok) {
       uint32_t md = sm.p_mode[pj];
       const uint32_t c0 = sm.p_c0[pj], aux = sm.p_aux[pj];
@@ -1792,7 +1764,6 @@ __device__ __forceinline__ void expand_lean(const KArgs& a, const StepView& v, u
         // the child's label: its first token, and whether it closes a key
         cnode = c0 + q;
         const uint32_t lw = a.labels[cnode];
-        if (!queued) ++my_children;
         ftok = lw & kTokMask;
         have_child = true;
         label_sel = (lw & kSlotSel) && depth_ok;
@@ -2372,10 +2343,15 @@ __device__ __forceinline__ void helper_loop(const KArgs& a, const DevReq& d, uin
       sm.lq_sel = 0;
     }
     __syncthreads();
-    if constexpr (kLean)
-      expand_lean(a, sv, W, g * (uint32_t)kWaves, a.wgs * (uint32_t)kWaves, false, false,
-                  hashed, sm);
-    else
+    bool expanded = false;
+    if constexpr (kLean) {
+      if (queued) {
+        expand_queued(a, sv, W, g * (uint32_t)kWaves, a.wgs * (uint32_t)kWaves, false, false,
+                      hashed, sm);
+        expanded = true;
+      }
+    }
+    if (!expanded)
       expand_range(a, sv, W, g * (uint32_t)kWaves, a.wgs * (uint32_t)kWaves, false, false,
                    hashed, sm);
     // the row lookups are done: empty the hash for the next step
@@ -2737,13 +2713,16 @@ __device__ __forceinline__ void tiny_steps(
 // one's start and output.
 // kLean: every beam and row of the launch is at most kBlock long (launch_tbs
 // is told), so that the parent table and the row of a step are always in LDS,
-// one thread an entry.  The instantiation leaves out the code for longer ones
-// and queues the items of large steps: 103 KB of code against 117 KB with
-// neither, which pays at every step since the leader's loop does not fit the
-// 64 KB instruction cache (the queue beside the general code made calls of
-// batch 1 3-5% slower).  The general one shares the functions but not the text
-// of a step's expansion (expand_range, expand_lean): small calls are as fast
-// with it as they were without the lean one.
+// one thread an entry.  The instantiation leaves out most of the code for longer
+// ones and queues the items of large steps (expand_queued beside expand_range):
+// 122 KB of code against the general one's 117.  An instantiation of its own,
+// since the leader's loop does not fit the 64 KB instruction cache: with the
+// queue in the general code calls of batch 1 were 3-5% slower.  The two share
+// their functions but not the text of a step's expansion below, which cost the
+// general one 1-2% as a common one.  (One item loop for queued and other steps
+// made the lean one's small steps ~1 us slower each, 46.0 -> 41.7 us a staged
+// request of long keys that hardly any proposal continues, and batch 64 at beam
+// = K = 1000 663 -> 638 us a call.)
 template <bool kLouds, bool kStreamed, bool kLean>
 __global__ void __launch_bounds__(kBlock) tbs_kernel(KArgs a) {
   __shared__ SmemOf<kLean> sm;
@@ -2790,9 +2769,8 @@ __global__ void __launch_bounds__(kBlock) tbs_kernel(KArgs a) {
   const uint8_t* in = a.stage + uni(d.in_off);
   const double* lnf = (const double*)in;
   const uint32_t* beams = (const uint32_t*)(in + d.beams_off);
-  // (the lean instantiation: in scalar registers, for want of others)
-  const uint32_t* rid = (const uint32_t*)(in + (kLean ? uni(d.rid_off) : d.rid_off));
-  const float* rlp = (const float*)(in + (kLean ? uni(d.rlp_off) : d.rlp_off));
+  const uint32_t* rid = (const uint32_t*)(in + d.rid_off);
+  const float* rlp = (const float*)(in + d.rlp_off);
   // the proposals' indices in the caller's rows, when some row came out of
   // order (else index = position)
   const uint16_t* rk = ss.rk ? (const uint16_t*)(in + d.rk_off) : nullptr;
@@ -2827,14 +2805,15 @@ __global__ void __launch_bounds__(kBlock) tbs_kernel(KArgs a) {
   uint32_t gen = 0;
   unsigned long long t_post = 0;  // (thread 0) wall clock of the last post
 
-  // Instantiations whose registers are full keep thread 0's clocks and the
-  // candidates in LDS and form the addresses of loops where they are used
-  // (thread_idx).  In the streamed search that takes 95.2 -> 93.3 us of device
-  // time at beam 500, batch 1 over 10M keys; the staged one, with fewer live
-  // values, loses by it: 91.8 -> 95.3 us a request at beam 250, launches of 32.
-  constexpr bool kTight = kLean || kStreamed;
+  // kLdsClocks: thread 0's clocks and the candidates in LDS.  kTight: addresses
+  // of loops are formed where they are used (thread_idx).  In the streamed
+  // search the two take 95.2 -> 93.3 us of device time at beam 500, batch 1 over
+  // 10M keys; the staged one, with fewer live values, loses by the clocks: 91.8
+  // -> 95.3 us a request at beam 250, launches of 32.  The lean instantiations
+  // need the second for their registers.
+  constexpr bool kLdsClocks = kStreamed, kTight = kLean || kStreamed;
   unsigned long long t_exp = 0, t_sel = 0, t_all0 = wall_clock64();
-  if constexpr (kTight) {
+  if constexpr (kLdsClocks) {
     if (tid == 0) sm.t_all0 = t_all0;
   }
   // per-step profile rows after the output tokens: kStepStats u64 per step
@@ -2845,7 +2824,7 @@ __global__ void __launch_bounds__(kBlock) tbs_kernel(KArgs a) {
     sm.status = 0;
     sm.multi_item = 0;
     sm.cnt_parents = sm.cnt_children = sm.cnt_probes = 0;
-    if constexpr (kTight) sm.t_exp = sm.t_sel = sm.n_cands = 0;
+    if constexpr (kLdsClocks) sm.t_exp = sm.t_sel = sm.n_cands = 0;
   }
   uint32_t n_cur = 1, nS = 0, hist_used = 0;
   uint64_t n_cands = 0;
@@ -2928,7 +2907,7 @@ __global__ void __launch_bounds__(kBlock) tbs_kernel(KArgs a) {
           n_cur = sm.tiny_ncur;
           nS = sm.tiny_nS;
           hist_used = sm.tiny_hist;
-          if constexpr (kTight) {
+          if constexpr (kLdsClocks) {
             if (tid == 0) {
               lds_add(&sm.n_cands, sm.tiny_cands);
               lds_add(&sm.t_exp, sm.tiny_ticks);
@@ -3056,7 +3035,7 @@ __global__ void __launch_bounds__(kBlock) tbs_kernel(KArgs a) {
       }
     }
     if (tid == 0) {
-      if constexpr (kTight) lds_add(&sm.cnt_parents, n_cur);
+      if constexpr (kLdsClocks) lds_add(&sm.cnt_parents, n_cur);
       else sm.cnt_parents += n_cur;
       // this workgroup's expansion counters (expand_range of the leader
       // relies on them being zero)
@@ -3096,8 +3075,7 @@ __global__ void __launch_bounds__(kBlock) tbs_kernel(KArgs a) {
     sv.cut = 0.0;
     sv.cut_mode = kCutNone;
     uint32_t sh_next = 0, sh_sel = 0;  // (shared) the pushes of the step
-    // The step's expansion, of the two instantiations apart (see expand_lean):
-    // one text for both cost the general one's small calls 1-2%.
+    // The step's expansion, of the two instantiations apart (see kLean).
     if constexpr (!kLean) {
       if (shared) {
         // publish the step (the helpers read the row from the staged request),
@@ -3117,7 +3095,7 @@ __global__ void __launch_bounds__(kBlock) tbs_kernel(KArgs a) {
         ++gen;
         if (tid == 0) {
           st_dev(&ctl->go, tag | gen);
-          if constexpr (kTight) sm.t_post = wall_clock64();
+          if constexpr (kLdsClocks) sm.t_post = wall_clock64();
           else t_post = wall_clock64();
         }
       }
@@ -3144,7 +3122,7 @@ __global__ void __launch_bounds__(kBlock) tbs_kernel(KArgs a) {
         // not running.  Then every claimed slice is waited for: a helper that
         // claimed one is running and finishes it.
         unsigned long long tw0 = 0;
-        if constexpr (!kTight) tw0 = wall_clock64();
+        if constexpr (!kLdsClocks) tw0 = wall_clock64();
         else if (tid == 0) sm.t_wait = wall_clock64();
         const unsigned long long mygo = tag | gen;
         unsigned long long* claims = (unsigned long long*)(ws + a.lay.claims);
@@ -3157,7 +3135,7 @@ __global__ void __launch_bounds__(kBlock) tbs_kernel(KArgs a) {
             pending_any = false;
             break;
           }
-          if constexpr (kTight) t_post = sm.t_post;
+          if constexpr (kLdsClocks) t_post = sm.t_post;
           if (tid == 0) sm.lead_flag = (wall_clock64() - t_post > kGraceTicks) ? 1u : 0u;
           __syncthreads();
           const bool expired = sm.lead_flag != 0;
@@ -3217,7 +3195,7 @@ __global__ void __launch_bounds__(kBlock) tbs_kernel(KArgs a) {
           if (!all_done) sm.status |= kStatusCorrupt;
           if (t < d.out_T) {
             uint64_t* row = step_stats + (uint64_t)t * kStepStats;
-            if constexpr (kTight) tw0 = sm.t_wait;
+            if constexpr (kLdsClocks) tw0 = sm.t_wait;
             row[8] = tw1 - tw0;
             row[9] = wall_clock64() - tw1;
           }
@@ -3295,8 +3273,12 @@ __global__ void __launch_bounds__(kBlock) tbs_kernel(KArgs a) {
         }
         const unsigned long long mygo = tag | gen;
         for (uint32_t taken = 0, slice = 0;;) {
-          expand_lean(a, sv, W, slice * (uint32_t)kWaves,
-                      (shared ? a.wgs : 1u) * (uint32_t)kWaves, true, !shared, hashed, sm);
+          if (sv.queued)
+            expand_queued(a, sv, W, slice * (uint32_t)kWaves,
+                          (shared ? a.wgs : 1u) * (uint32_t)kWaves, true, !shared, hashed, sm);
+          else
+            expand_range(a, sv, W, slice * (uint32_t)kWaves,
+                         (shared ? a.wgs : 1u) * (uint32_t)kWaves, true, !shared, hashed, sm);
           lead_ch += sm.w_children;
           lead_pr += sm.w_probes;
           if (!shared) break;
@@ -3424,9 +3406,9 @@ __global__ void __launch_bounds__(kBlock) tbs_kernel(KArgs a) {
     // 0 adds the overflow bit below, which every thread derives itself
     const bool overflow = n_next > next_cap || nS + n_new > sel_cap;
     const bool stop = overflow || sm.status != 0;
-    if constexpr (!kTight) n_cands += (uint64_t)n_next + n_new;
+    if constexpr (!kLdsClocks) n_cands += (uint64_t)n_next + n_new;
     if (tid == 0) {
-      if constexpr (kTight) {
+      if constexpr (kLdsClocks) {
         lds_add(&sm.n_cands, (uint64_t)n_next + n_new);
         lds_add(&sm.cnt_children, w_ch);
         lds_add(&sm.cnt_probes, w_pr);
@@ -3441,7 +3423,7 @@ __global__ void __launch_bounds__(kBlock) tbs_kernel(KArgs a) {
       break;
     }
     const unsigned long long t1 = wall_clock64();
-    if constexpr (!kTight) t_exp += t1 - t0;
+    if constexpr (!kLdsClocks) t_exp += t1 - t0;
     else if (tid == 0) lds_add(&sm.t_exp, t1 - t0);
     if (tid == 0 && t < d.out_T) {
       uint64_t* row = step_stats + (uint64_t)t * kStepStats;
@@ -3565,7 +3547,7 @@ __global__ void __launch_bounds__(kBlock) tbs_kernel(KArgs a) {
       }
     }
     if (stop_after) {
-      if constexpr (!kTight) t_sel += wall_clock64() - t1;
+      if constexpr (!kLdsClocks) t_sel += wall_clock64() - t1;
       else if (tid == 0) lds_add(&sm.t_sel, wall_clock64() - t1);
       break;
     }
@@ -3772,7 +3754,7 @@ __global__ void __launch_bounds__(kBlock) tbs_kernel(KArgs a) {
       cur_which ^= 1u;
     }
     par_ready = next_table;
-    if constexpr (!kTight) t_sel += wall_clock64() - t1;
+    if constexpr (!kLdsClocks) t_sel += wall_clock64() - t1;
     else if (tid == 0) lds_add(&sm.t_sel, wall_clock64() - t1);
   }
   // release the helpers
@@ -3890,7 +3872,7 @@ __global__ void __launch_bounds__(kBlock) tbs_kernel(KArgs a) {
   if (tid == 0) {
     oh->count = status ? 0 : nS;
     const unsigned long long tend = wall_clock64();
-    if constexpr (kTight) {
+    if constexpr (kLdsClocks) {
       t_exp = sm.t_exp;
       t_sel = sm.t_sel;
       t_all0 = sm.t_all0;
