@@ -2713,16 +2713,15 @@ __device__ __forceinline__ void tiny_steps(
 // one's start and output.
 // kLean: every beam and row of the launch is at most kBlock long (launch_tbs
 // is told), so that the parent table and the row of a step are always in LDS,
-// one thread an entry.  The instantiation leaves out most of the code for longer
-// ones and queues the items of large steps (expand_queued beside expand_range):
-// 122 KB of code against the general one's 117.  An instantiation of its own,
-// since the leader's loop does not fit the 64 KB instruction cache: with the
-// queue in the general code calls of batch 1 were 3-5% slower.  The two share
-// their functions but not the text of a step's expansion below, which cost the
-// general one 1-2% as a common one.  (One item loop for queued and other steps
-// made the lean one's small steps ~1 us slower each, 46.0 -> 41.7 us a staged
-// request of long keys that hardly any proposal continues, and batch 64 at beam
-// = K = 1000 663 -> 638 us a call.)
+// one thread an entry.  The instantiation queues the items of large steps and
+// cuts their pushes (expand_queued, cut_of_step), beside the general code for
+// every other step: 133 KB of code against the general one's 117.  An
+// instantiation of its own, since the leader's loop does not fit the 64 KB
+// instruction cache: with the queue in the general one calls of batch 1 were 3-5%
+// slower.  Its small steps run the general text, not a common loop of both
+// kinds, which made them up to 1 us slower each: a staged request of long keys
+// that hardly any proposal continues 46.0 -> 43.5 us, the streamed beam = K =
+// 1000, batch 4 over 800M keys 167.3 -> 164.1 us a call.
 template <bool kLouds, bool kStreamed, bool kLean>
 __global__ void __launch_bounds__(kBlock) tbs_kernel(KArgs a) {
   __shared__ SmemOf<kLean> sm;
@@ -3069,14 +3068,27 @@ __global__ void __launch_bounds__(kBlock) tbs_kernel(KArgs a) {
     sv.keep_lds_max = min((uint32_t)kPushCap, beams[t]);
     sv.one_each = (kLean || n_cur <= (uint32_t)kBlock) && sm.multi_item == 0;
 
-
     const bool shared = a.wgs > 1 && W >= a.share_min;
     sv.queued = false;
     sv.cut = 0.0;
     sv.cut_mode = kCutNone;
     uint32_t sh_next = 0, sh_sel = 0;  // (shared) the pushes of the step
-    // The step's expansion, of the two instantiations apart (see kLean).
-    if constexpr (!kLean) {
+    // The step's expansion, of queued and other steps apart (see kLean).
+    const bool hashed = (kLean || K <= kRowHashMaxK) && W >= kRowHashMinWork;
+    if constexpr (kLean) {
+      const uint32_t step_waves = (shared ? a.wgs : 1u) * (uint32_t)kWaves;
+      // (an item's place among its parent's fits the queue's 16 bits)
+      if (hashed && a.scan_limit <= 65536u) {
+        sv.queued = has_chunks(W, step_waves, kQueueMinChunks);
+        if (shared && (sv.queued || (beams[t] >= kCutMinBeam &&
+                                     has_chunks(W, step_waves, kCutMinChunks)))) {
+          cut_of_step(a, sv, W, step_waves, beams[t],
+                      (const uint64_t*)(in + d.kb_off) + 2ull * t, sm);
+          sv.queued = sv.queued || sv.cut_mode != kCutNone;
+        }
+      }
+    }
+    if (!kLean || !sv.queued) {
       if (shared) {
         // publish the step (the helpers read the row from the staged request),
         // then wake the helpers
@@ -3089,6 +3101,7 @@ __global__ void __launch_bounds__(kBlock) tbs_kernel(KArgs a) {
           st_dev(&ctl->sel_which, sel_which);
           st_dev(&ctl->cur_which, cur_which);
           st_dev(&ctl->hist_n, hist_used);
+          if constexpr (kLean) st_dev(&ctl->cut_mode, (uint32_t)kCutNone);
         }
         wait_stores();  // the step's data is complete before `go` moves
         __syncthreads();
@@ -3101,7 +3114,6 @@ __global__ void __launch_bounds__(kBlock) tbs_kernel(KArgs a) {
       }
       // (the parent table ended synchronised: the row and the emptied hash are
       // visible)
-      const bool hashed = K <= kRowHashMaxK && W >= kRowHashMinWork;
       if (hashed) hash_row<false>(K, sm);
       // (streamed) helper 1 copying the request's later rows claims no slice
       // meanwhile: its slice is taken over at once rather than after the
@@ -3216,115 +3228,158 @@ __global__ void __launch_bounds__(kBlock) tbs_kernel(KArgs a) {
           if (wp) atomicAdd(&sm.w_probes, wp);
         }
       }
-    } else {
-      const bool hashed = W >= kRowHashMinWork;
-      const uint32_t step_waves = (shared ? a.wgs : 1u) * (uint32_t)kWaves;
-      // (an item's place among its parent's fits the queue's 16 bits)
-      if (hashed && a.scan_limit <= 65536u) {
-        sv.queued = has_chunks(W, step_waves, kQueueMinChunks);
-        if (shared && (sv.queued || (beams[t] >= kCutMinBeam &&
-                                     has_chunks(W, step_waves, kCutMinChunks)))) {
-          cut_of_step(a, sv, W, step_waves, beams[t], (const uint64_t*)(in + d.kb_off) + 2ull * t, sm);
-          sv.queued = sv.queued || sv.cut_mode != kCutNone;
-        }
-      }
-      // the leader's slice 0, then (shared) the slices it takes over: one call
-      // of the inlined expansion for both, which keeps its code and registers
-      // to one copy
-      uint32_t lead_ch = 0, lead_pr = 0;  // the counters of the leader's slices
-      uint32_t n_stolen = 0;
-      bool stole = false;  // (thread i) slice i + 1 was taken over here
-      const uint32_t nh = a.wgs - 1;  // helper slots 1 .. nh (nh < kBlock)
-      // one round, or two when a cut let too few pushes through
-      for (;;) {
-        if (shared) {
-          // publish the step (the helpers read the row from the staged request),
-          // then wake the helpers
-          if (tid == 0) {
-            if (sv.cut_mode != kCutBelow) st_dev(&ctl->pushes, 0ull);
-            st_dev(&ctl->t, t);
-            st_dev(&ctl->W, W);
-            st_dev(&ctl->n_par, n_cur);
-            st_dev(&ctl->nS, nS);
-            st_dev(&ctl->sel_which, sel_which);
-            st_dev(&ctl->cur_which, cur_which);
-            st_dev(&ctl->hist_n, hist_used);
-            st_dev(&ctl->cut, (unsigned long long)__double_as_longlong(sv.cut));
-            st_dev(&ctl->cut_mode, sv.cut_mode | (sv.queued ? kStepQueued : 0u));
+    }
+    if constexpr (kLean) {
+      if (sv.queued) {
+        // the leader's slice 0, then (shared) the slices it takes over: one call
+        // of the inlined expansion for both, which keeps its code and registers
+        // to one copy
+        uint32_t lead_ch = 0, lead_pr = 0;  // the counters of the leader's slices
+        uint32_t n_stolen = 0;
+        bool stole = false;  // (thread i) slice i + 1 was taken over here
+        const uint32_t nh = a.wgs - 1;  // helper slots 1 .. nh (nh < kBlock)
+        // one round, or two when a cut let too few pushes through
+        for (;;) {
+          if (shared) {
+            // publish the step (the helpers read the row from the staged request),
+            // then wake the helpers
+            if (tid == 0) {
+              if (sv.cut_mode != kCutBelow) st_dev(&ctl->pushes, 0ull);
+              st_dev(&ctl->t, t);
+              st_dev(&ctl->W, W);
+              st_dev(&ctl->n_par, n_cur);
+              st_dev(&ctl->nS, nS);
+              st_dev(&ctl->sel_which, sel_which);
+              st_dev(&ctl->cur_which, cur_which);
+              st_dev(&ctl->hist_n, hist_used);
+              st_dev(&ctl->cut, (unsigned long long)__double_as_longlong(sv.cut));
+              st_dev(&ctl->cut_mode, sv.cut_mode | kStepQueued);
+            }
+            wait_stores();  // the step's data is complete before `go` moves
+            __syncthreads();
+            ++gen;
+            if (tid == 0) {
+              st_dev(&ctl->go, tag | gen);
+              sm.t_post = wall_clock64();
+            }
           }
-          wait_stores();  // the step's data is complete before `go` moves
-          __syncthreads();
-          ++gen;
-          if (tid == 0) {
-            st_dev(&ctl->go, tag | gen);
-            sm.t_post = wall_clock64();
+          // (the parent table ended synchronised: the row and the emptied hash are
+          // visible)
+          if (sv.cut_mode != kCutBelow) hash_row<true>(K, sm);
+          // (streamed) helper 1 copying the request's later rows claims no slice
+          // meanwhile: its slice is taken over at once rather than after the
+          // grace period (thread 0 stands for slot 1 below)
+          bool copying1 = false;
+          if constexpr (kStreamed) {
+            if (shared && tid == 0 && !ss.done && !ss.own && ss.split < T)
+              copying1 = ld_relaxed(&ctl->copy) == (tag | kCopyClaimed);
           }
-        }
-        // (the parent table ended synchronised: the row and the emptied hash are
-        // visible)
-        if (hashed && sv.cut_mode != kCutBelow) hash_row<true>(K, sm);
-        // (streamed) helper 1 copying the request's later rows claims no slice
-        // meanwhile: its slice is taken over at once rather than after the
-        // grace period (thread 0 stands for slot 1 below)
-        bool copying1 = false;
-        if constexpr (kStreamed) {
-          if (shared && tid == 0 && !ss.done && !ss.own && ss.split < T)
-            copying1 = ld_relaxed(&ctl->copy) == (tag | kCopyClaimed);
-        }
-        const unsigned long long mygo = tag | gen;
-        for (uint32_t taken = 0, slice = 0;;) {
-          if (sv.queued)
+          const unsigned long long mygo = tag | gen;
+          for (uint32_t taken = 0, slice = 0;;) {
             expand_queued(a, sv, W, slice * (uint32_t)kWaves,
                           (shared ? a.wgs : 1u) * (uint32_t)kWaves, true, !shared, hashed, sm);
-          else
-            expand_range(a, sv, W, slice * (uint32_t)kWaves,
-                         (shared ? a.wgs : 1u) * (uint32_t)kWaves, true, !shared, hashed, sm);
-          lead_ch += sm.w_children;
-          lead_pr += sm.w_probes;
-          if (!shared) break;
-          if (slice == 0) {
-            // The helpers' slices: each is claimed by its helper (its claim word
-            // set to this step) or, once kGraceTicks have passed since the post,
-            // taken over here -- so the step never waits for a workgroup that is
-            // not running.  Then every claimed slice is waited for: a helper that
-            // claimed one is running and finishes it.
-            if (tid == 0) sm.t_wait = wall_clock64();
-            unsigned long long* claims = (unsigned long long*)(ws + a.lay.claims);
-            bool pending_any = true;
-            for (;;) {
-              const int pending = __syncthreads_count(tid < nh && !copying1 &&
-                                                      ld_relaxed(&claims[tid + 1]) != mygo);
-              if (pending == 0) {
-                pending_any = false;
-                break;
+            lead_ch += sm.w_children;
+            lead_pr += sm.w_probes;
+            if (!shared) break;
+            if (slice == 0) {
+              // The helpers' slices: each is claimed by its helper (its claim word
+              // set to this step) or, once kGraceTicks have passed since the post,
+              // taken over here -- so the step never waits for a workgroup that is
+              // not running.  Then every claimed slice is waited for: a helper that
+              // claimed one is running and finishes it.
+              if (tid == 0) sm.t_wait = wall_clock64();
+              unsigned long long* claims = (unsigned long long*)(ws + a.lay.claims);
+              bool pending_any = true;
+              for (;;) {
+                const int pending = __syncthreads_count(tid < nh && !copying1 &&
+                                                        ld_relaxed(&claims[tid + 1]) != mygo);
+                if (pending == 0) {
+                  pending_any = false;
+                  break;
+                }
+                if (tid == 0) sm.lead_flag = (wall_clock64() - sm.t_post > kGraceTicks) ? 1u : 0u;
+                __syncthreads();
+                const bool expired = sm.lead_flag != 0;
+                __syncthreads();
+                if (expired) break;
+                __builtin_amdgcn_s_sleep(2);
               }
-              if (tid == 0) sm.lead_flag = (wall_clock64() - sm.t_post > kGraceTicks) ? 1u : 0u;
-              __syncthreads();
-              const bool expired = sm.lead_flag != 0;
-              __syncthreads();
-              if (expired) break;
-              __builtin_amdgcn_s_sleep(2);
+              // (thread 0 alone knows whether helper 1 is copying: the takeover
+              // runs when any slot is still pending or helper 1 copies)
+              if (__syncthreads_or(pending_any || copying1)) {
+                if (tid == 0) sm.n_stolen = 0;
+                __syncthreads();
+                // raise every unclaimed word (helper 1's alone when only it is
+                // copying): a slice whose word this raises is taken over here; one
+                // a helper raised first stays the helper's
+                if (tid < nh && (pending_any || tid == 0) &&
+                    atomicMax(&claims[tid + 1], mygo) < mygo) {
+                  stole = true;
+                  const uint32_t k = atomicAdd(&sm.n_stolen, 1u);
+                  sm.stolen[k] = (uint16_t)(tid + 1);
+                }
+                __syncthreads();
+                n_stolen = sm.n_stolen;
+              }
             }
-            // (thread 0 alone knows whether helper 1 is copying: the takeover
-            // runs when any slot is still pending or helper 1 copies)
-            if (__syncthreads_or(pending_any || copying1)) {
-              if (tid == 0) sm.n_stolen = 0;
-              __syncthreads();
-              // raise every unclaimed word (helper 1's alone when only it is
-              // copying): a slice whose word this raises is taken over here; one
-              // a helper raised first stays the helper's
-              if (tid < nh && (pending_any || tid == 0) &&
-                  atomicMax(&claims[tid + 1], mygo) < mygo) {
-                stole = true;
-                const uint32_t k = atomicAdd(&sm.n_stolen, 1u);
-                sm.stolen[k] = (uint16_t)(tid + 1);
-              }
-              __syncthreads();
-              n_stolen = sm.n_stolen;
+            if (taken == n_stolen) break;
+            slice = sm.stolen[taken++];
+            __syncthreads();
+            if (tid == 0) {
+              sm.w_children = 0;
+              sm.w_probes = 0;
+              sm.lq_next = 0;
+              sm.lq_sel = 0;
+            }
+            __syncthreads();
+          }
+          if (!shared) break;
+          // Every slice a helper claimed: thread i waits for helper i + 1's done
+          // word to carry this step's tag (written after its pushes and its
+          // counters are complete), unless thread i took that slice over.
+          const unsigned long long tw1 = wall_clock64();
+          unsigned long long* dones = (unsigned long long*)(ws + a.lay.dones);
+          const bool waits = tid < nh && !stole;
+          bool all_done = false;
+          for (uint32_t it = 0; it < kSpinLimit; ++it) {
+            if (__syncthreads_count(waits && ld_relaxed(&dones[2 * (tid + 1)]) != mygo) == 0) {
+              all_done = true;
+              break;
+            }
+            __builtin_amdgcn_s_sleep(1);
+          }
+          if (tid == 0) {
+            if (!all_done) sm.status |= kStatusCorrupt;
+            if (t < d.out_T) {
+              uint64_t* row = step_stats + (uint64_t)t * kStepStats;
+              // (the sums of a step's rounds; the rows start at 0)
+              row[8] += tw1 - sm.t_wait;
+              row[9] += wall_clock64() - tw1;
             }
           }
-          if (taken == n_stolen) break;
-          slice = sm.stolen[taken++];
+          // the helpers' counters and the step's push counts, read together
+          const unsigned long long cw = waits ? ld_relaxed(&dones[2 * (tid + 1) + 1]) : 0ull;
+          const unsigned long long pw = ld_relaxed(&ctl->pushes);
+          sh_next = (uint32_t)pw;
+          sh_sel = (uint32_t)(pw >> 32);
+          const uint32_t wc = wave_sum((uint32_t)cw), wp = wave_sum((uint32_t)(cw >> 32));
+          if (tid == 0) {
+            sm.w_children = lead_ch;
+            sm.w_probes = lead_pr;
+          }
+          __syncthreads();
+          if ((tid & 63u) == 0u) {
+            if (wc) atomicAdd(&sm.w_children, wc);
+            if (wp) atomicAdd(&sm.w_probes, wp);
+          }
+          if (sv.cut_mode != kCutAbove || sh_next >= beams[t] || !all_done) break;
+          // too few pushes reach the cut: the others, in a second round
+          sv.cut_mode = kCutBelow;
+          __syncthreads();
+          lead_ch = sm.w_children;
+          lead_pr = sm.w_probes;
+          n_stolen = 0;
+          stole = false;
           __syncthreads();
           if (tid == 0) {
             sm.w_children = 0;
@@ -3332,61 +3387,6 @@ __global__ void __launch_bounds__(kBlock) tbs_kernel(KArgs a) {
             sm.lq_next = 0;
             sm.lq_sel = 0;
           }
-          __syncthreads();
-        }
-        if (!shared) break;
-        // Every slice a helper claimed: thread i waits for helper i + 1's done
-        // word to carry this step's tag (written after its pushes and its
-        // counters are complete), unless thread i took that slice over.
-        const unsigned long long tw1 = wall_clock64();
-        unsigned long long* dones = (unsigned long long*)(ws + a.lay.dones);
-        const bool waits = tid < nh && !stole;
-        bool all_done = false;
-        for (uint32_t it = 0; it < kSpinLimit; ++it) {
-          if (__syncthreads_count(waits && ld_relaxed(&dones[2 * (tid + 1)]) != mygo) == 0) {
-            all_done = true;
-            break;
-          }
-          __builtin_amdgcn_s_sleep(1);
-        }
-        if (tid == 0) {
-          if (!all_done) sm.status |= kStatusCorrupt;
-          if (t < d.out_T) {
-            uint64_t* row = step_stats + (uint64_t)t * kStepStats;
-            // (the sums of a step's rounds; the rows start at 0)
-            row[8] += tw1 - sm.t_wait;
-            row[9] += wall_clock64() - tw1;
-          }
-        }
-        // the helpers' counters and the step's push counts, read together
-        const unsigned long long cw = waits ? ld_relaxed(&dones[2 * (tid + 1) + 1]) : 0ull;
-        const unsigned long long pw = ld_relaxed(&ctl->pushes);
-        sh_next = (uint32_t)pw;
-        sh_sel = (uint32_t)(pw >> 32);
-        const uint32_t wc = wave_sum((uint32_t)cw), wp = wave_sum((uint32_t)(cw >> 32));
-        if (tid == 0) {
-          sm.w_children = lead_ch;
-          sm.w_probes = lead_pr;
-        }
-        __syncthreads();
-        if ((tid & 63u) == 0u) {
-          if (wc) atomicAdd(&sm.w_children, wc);
-          if (wp) atomicAdd(&sm.w_probes, wp);
-        }
-        if (sv.cut_mode != kCutAbove || sh_next >= beams[t] || !all_done) break;
-        // too few pushes reach the cut: the others, in a second round
-        sv.cut_mode = kCutBelow;
-        __syncthreads();
-        lead_ch = sm.w_children;
-        lead_pr = sm.w_probes;
-        n_stolen = 0;
-        stole = false;
-        __syncthreads();
-        if (tid == 0) {
-          sm.w_children = 0;
-          sm.w_probes = 0;
-          sm.lq_next = 0;
-          sm.lq_sel = 0;
         }
       }
       if (a.step_kinds && tid == 0 && t < d.out_T)
